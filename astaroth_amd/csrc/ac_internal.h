@@ -73,6 +73,7 @@ struct SubstepArgs {
     const AcReal* __restrict__ cin[NF];
     AcReal* __restrict__ cout[NF];
     int mx, my, mz, mxy;
+    long stride; // cells from each field of `in` to the next, and of `out` to the next
     int3 start, end;
     // 1: the tile halos and the planes beyond the interior are read at their periodic images
     // inside the interior, so no ghost cell is read (configurations of kernel_config_reads_images)
@@ -111,9 +112,6 @@ hipError_t launch_substep_batch(int tile_x, int tile_y, const SubstepArgs* boxes
 int kernel_config_count();
 AcKernelConfig kernel_config_at(int index);
 AcKernelConfig default_kernel_config(int nx, int ny, int nz);
-// z-depth of equal z-chunks for a z-march of tile_x x tile_y columns with `blocks_per_cu` blocks
-// resident per CU (0: whole columns), chosen by the launch's rounds of resident blocks.
-int balanced_z_depth(int nx, int ny, int nz, int tile_x, int tile_y, int blocks_per_cu);
 
 // Periodic fill of the ghost cells inside [start, end) of `nfields` buffers (boundconds.hip).
 hipError_t launch_periodic_fill(AcReal* const* fields, int nfields, int nx, int ny, int nz,
@@ -167,6 +165,9 @@ struct device_s {
     AcMeshInfo uniforms;     // parameters the kernels use (the reference's d_mesh_info)
     hipStream_t streams[NUM_STREAMS];
     ac::VertexBufferArray vba;
+    AcReal* field_sets[2]; // the allocations behind vba (in and out at creation), and, compensated
+    AcReal* comp_sets[2];  // integration only, behind comp
+    long field_stride;     // cells from one field of a set to the next
     double* reduce_partials;
     double* reduce_scratch; // this GPU's copy of the library's reduction scratch array
     double* reduce_result;

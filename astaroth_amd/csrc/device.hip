@@ -100,7 +100,8 @@ make_args(const Device d, const AcReal* const* in, AcReal* const* out, int step,
     a.mx    = nx_of(d) + 6;
     a.my    = ny_of(d) + 6;
     a.mz    = nz_of(d) + 6;
-    a.mxy   = a.mx * a.my;
+    a.mxy    = a.mx * a.my;
+    a.stride = d->field_stride;
     a.start = start;
     a.end   = end;
     a.wrap  = 0;
@@ -493,14 +494,19 @@ acDeviceCreate(const int id, const AcMeshInfo config, Device* device_handle)
     d->halo_buffer_len = 0;
     for (int q = 0; q < NF; ++q)
         d->comp[0][q] = d->comp[1][q] = nullptr;
+    d->comp_sets[0] = d->comp_sets[1] = nullptr;
     for (int i = 0; i < NUM_STREAMS; ++i)
         AC_HIP_CHECK(hipStreamCreateWithFlags(&d->streams[i], hipStreamNonBlocking));
 
     const size_t m     = (size_t)(nx + 6) * (ny + 6) * (nz + 6);
-    const size_t bytes = m * sizeof(AcReal);
+    // one allocation per set, its fields equally spaced: the solve then needs one base and one
+    // stride instead of a pointer per field
+    d->field_stride = (long)((m * sizeof(AcReal) + 255) / 256 * 256 / sizeof(AcReal));
+    for (int set = 0; set < 2; ++set)
+        AC_HIP_CHECK(hipMalloc((void**)&d->field_sets[set], NF * d->field_stride * sizeof(AcReal)));
     for (int q = 0; q < NF; ++q) {
-        AC_HIP_CHECK(hipMalloc((void**)&d->vba.in[q], bytes));
-        AC_HIP_CHECK(hipMalloc((void**)&d->vba.out[q], bytes));
+        d->vba.in[q]  = d->field_sets[0] + q * d->field_stride;
+        d->vba.out[q] = d->field_sets[1] + q * d->field_stride;
         AC_HIP_CHECK(launch_fill_constant(d->vba.in[q], (long)m, AcReal(0), d->streams[0]));
         AC_HIP_CHECK(launch_fill_constant(d->vba.out[q], (long)m, AcReal(0), d->streams[0]));
         d->base_in[q] = d->vba.in[q];
@@ -533,10 +539,8 @@ acDeviceDestroy(Device device)
     AC_HIP_CHECK(hipSetDevice(device->id));
     AC_HIP_CHECK(hipDeviceSynchronize());
     invalidate_graphs(device);
-    for (int q = 0; q < NF; ++q) {
-        AC_HIP_CHECK(hipFree(device->vba.in[q]));
-        AC_HIP_CHECK(hipFree(device->vba.out[q]));
-    }
+    for (int set = 0; set < 2; ++set)
+        AC_HIP_CHECK(hipFree(device->field_sets[set]));
     AC_HIP_CHECK(hipFree(device->reduce_partials));
     AC_HIP_CHECK(hipFree(device->reduce_result));
     AC_HIP_CHECK(hipHostFree(device->reduce_result_host));
@@ -546,9 +550,8 @@ acDeviceDestroy(Device device)
     if (device->halo_buffer)
         AC_HIP_CHECK(hipFree(device->halo_buffer));
     for (int set = 0; set < 2; ++set)
-        for (int q = 0; q < NF; ++q)
-            if (device->comp[set][q])
-                AC_HIP_CHECK(hipFree(device->comp[set][q]));
+        if (device->comp_sets[set])
+            AC_HIP_CHECK(hipFree(device->comp_sets[set]));
     for (int i = 0; i < NUM_STREAMS; ++i)
         AC_HIP_CHECK(hipStreamDestroy(device->streams[i]));
     delete device;
@@ -1414,19 +1417,21 @@ acDeviceSetCompensatedIntegration(const Device device, const int enable)
     AC_HIP_CHECK(hipDeviceSynchronize());
     const bool on = device->comp[0][0] != nullptr;
     if (enable && !on) {
-        const size_t bytes = acVertexBufferSizeBytes(device->local_config);
-        for (int set = 0; set < 2; ++set)
-            for (int q = 0; q < NF; ++q) {
-                AC_HIP_CHECK(hipMalloc((void**)&device->comp[set][q], bytes));
-                AC_HIP_CHECK(hipMemset(device->comp[set][q], 0, bytes));
-            }
+        const size_t bytes = NF * device->field_stride * sizeof(AcReal);
+        for (int set = 0; set < 2; ++set) {
+            AC_HIP_CHECK(hipMalloc((void**)&device->comp_sets[set], bytes));
+            AC_HIP_CHECK(hipMemset(device->comp_sets[set], 0, bytes));
+            for (int q = 0; q < NF; ++q)
+                device->comp[set][q] = device->comp_sets[set] + q * device->field_stride;
+        }
     }
     else if (!enable && on) {
-        for (int set = 0; set < 2; ++set)
-            for (int q = 0; q < NF; ++q) {
-                AC_HIP_CHECK(hipFree(device->comp[set][q]));
+        for (int set = 0; set < 2; ++set) {
+            AC_HIP_CHECK(hipFree(device->comp_sets[set]));
+            device->comp_sets[set] = nullptr;
+            for (int q = 0; q < NF; ++q)
                 device->comp[set][q] = nullptr;
-            }
+        }
     }
     invalidate_graphs(device);
     return AC_SUCCESS;

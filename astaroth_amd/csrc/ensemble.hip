@@ -343,7 +343,8 @@ build_args(Ensemble e, AcReal dt)
                 x.mx    = n.x + 6;
                 x.my    = n.y + 6;
                 x.mz    = n.z + 6;
-                x.mxy   = x.mx * x.my;
+                x.mxy    = x.mx * x.my;
+                x.stride = x.in[1] - x.in[0];
                 x.start = make_int3(NGHOST, NGHOST, NGHOST);
                 x.end   = make_int3(n.x + NGHOST, n.y + NGHOST, n.z + NGHOST);
                 x.wrap  = 1;
@@ -896,7 +897,8 @@ acEnsembleIntegrateStepLooped(Ensemble e, const AcReal dt)
             a.mx    = n.x + 6;
             a.my    = n.y + 6;
             a.mz    = n.z + 6;
-            a.mxy   = a.mx * a.my;
+            a.mxy    = a.mx * a.my;
+            a.stride = a.in[1] - a.in[0];
             a.start = make_int3(NGHOST, NGHOST, NGHOST);
             a.end   = make_int3(n.x + NGHOST, n.y + NGHOST, n.z + NGHOST);
             a.wrap  = images;

@@ -30,16 +30,18 @@
 //      per cell than variant 2; variant 4 is the same kernel compiled for two waves per SIMD.
 //  variants 7-12: the lean z-march with a 5-slot ring (7: one barrier per plane), or loading
 //      the previous stage before the next plane and storing each output plane at the start of
-//      the next step (8: 4 slots, the FP64 default; 9: 5 slots), and its two-waves-per-SIMD
+//      the next step (8: 4 slots, FP32; 9: 5 slots), and its two-waves-per-SIMD
 //      builds on 16 x 16 tiles (10: deferred stores; 11: previous stage first; 12: both).
 //  variant 13: variant 12 with an 8-phase plane loop (compile-time ring slots); 16: variant 12
 //      with a 5-slot ring.
-//  variants 17, 19, 22: variants 16, 12 and 10 with pinned LDS windows (every stencil read of a
-//      field's plane through one base register); 19 is the FP32 default.
+//  variants 17, 22: variants 16 and 10 with pinned LDS windows (every stencil read of a field's
+//      plane through one base register).
 //  variant 23: variant 17 loading each plane straight into its ring slot (direct-to-LDS loads).
 //  variants 5, 6: the lean z-march with a cell-major LDS ring (FP32; kept for comparison).
-//  The defaults also have builds that read the periodic images of the ghost cells (WRAP), used by
-//  the whole-step entry points of a periodic box where they are the faster form.
+//  variant 19 (FP32) and variant 8 on 16 x 16 tiles in FP64, the defaults: the ring march
+//      (solve_ring.h); variant 24: the FP32 ring march in 64 x 8 blocks whatever the box. The ring
+//      march can read the periodic images of the ghost cells (SubstepArgs::wrap), used by the
+//      whole-step entry points of a periodic box where that is the faster form.
 #include "physics.h"
 
 #include <algorithm>
@@ -1063,6 +1065,12 @@ struct ZMarchLean {
     }
 };
 
+} // namespace
+} // namespace ac
+#include "solve_ring.h"
+namespace ac {
+namespace {
+
 #if AC_DOUBLE_PRECISION == 0
 // ------------------------------------------------------------------------------------------
 // variants 5 and 6 (FP32): the lean z-march with a cell-major LDS ring
@@ -1675,6 +1683,9 @@ constexpr ConfigEntry kConfigs[] = {
     {23, 16, 16},
 #endif
     {8, 16, 16},
+#if AC_DOUBLE_PRECISION == 0
+    {24, 64, 8},
+#endif
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 
@@ -1698,6 +1709,17 @@ launch_zmarch_grid(ZMarchKernel kernel, const SubstepArgs& a, int zdepth, hipStr
     return hipGetLastError();
 }
 
+// Whether SubstepArgs::stride leads from each field to the next (what the ring march relies on).
+bool
+fields_equally_spaced(const SubstepArgs& a)
+{
+    for (int q = 1; q < NF; ++q)
+        if (a.in[q] - a.in[0] != q * a.stride || a.out[q] - a.out[0] != q * a.stride ||
+            (a.cin[0] && (a.cin[q] - a.cin[0] != q * a.stride || a.cout[q] - a.cout[0] != q * a.stride)))
+            return false;
+    return true;
+}
+
 template <int TX, int TY>
 hipError_t
 launch_direct(const SubstepArgs& a, hipStream_t stream)
@@ -1706,6 +1728,17 @@ launch_direct(const SubstepArgs& a, hipStream_t stream)
     const dim3 grid((nx + TX - 1) / TX, (ny + TY - 1) / TY, nz);
     solve_direct<TX, TY><<<grid, dim3(TX, TY), 0, stream>>>(a);
     return hipGetLastError();
+}
+
+
+template <int TX, int TY, int W, bool COMP>
+__global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W)))
+solve_ring(const SubstepArgs a, const int zdepth, const int ntx, const int nty)
+{
+    __shared__ typename ZMarchRing<TX, TY, COMP>::Shared sh;
+    int btx, bty, btz;
+    strip_tile(xcd_remap((int)blockIdx.x, (int)gridDim.x), ntx, nty, btx, bty, btz);
+    ring_column<TX, TY, COMP>(a, sh, btx, bty, a.start.z + btz * zdepth, zdepth);
 }
 
 } // namespace
@@ -1723,7 +1756,7 @@ kernel_config_supported(const AcKernelConfig& c)
 bool
 kernel_config_reads_images(const AcKernelConfig& c)
 {
-    // the defaults (FP32 variant 19, FP64 variant 8), compiled a second time with WRAP
+    // the ring march
 #if AC_DOUBLE_PRECISION == 1
     return c.variant == 8 && c.tile_x == 16 && c.tile_y == 16 && c.z_depth >= 0;
 #else
@@ -1734,17 +1767,13 @@ kernel_config_reads_images(const AcKernelConfig& c)
 bool
 default_reads_images(int nx, int ny, int nz)
 {
-    // The WRAP builds save the three fills of a step, but their launches slow down with the box
-    // (the far-side halo and plane reads: at 1024^3 FP32 a launch takes 51 ms against 36 ms
-    // with fills). Per step, fill + launch against images (ms, interleaved on one box):
-    //   FP64  384^3 13.15 / 13.02   512^3 29.37 / 29.53   768^3 100.0 / 105.1   1024^3 230 / 240
-    //   FP32  256^3 1.67 / 1.58     384^3 6.31 / 6.36     448^3 10.24 / 10.18   512^3 12.78 / 13.44
-    // so images below 512^3 cells in FP64 and below 384^3 in FP32.
-#if AC_DOUBLE_PRECISION == 1
+    // Reading images saves the three fills of a step but slows the launches down as the box grows
+    // (the far-side halo and plane reads). Per step, images against fills (ms, sustained):
+    //   FP32  128^3 0.176 / 0.201   256^3 1.45 / 1.47   384^3 4.93 / 5.04   448^3 7.91 / 8.06
+    //         512^3 11.80 / 11.40
+    //   FP64  128^3 0.406 / 0.458   256^3 3.08 / 3.20   384^3 10.85 / 11.04   512^3 25.07 / 25.16
+    // so images below 512^3 cells.
     return (double)nx * ny * nz < 512.0 * 512.0 * 512.0;
-#else
-    return (double)nx * ny * nz < 384.0 * 384.0 * 384.0;
-#endif
 }
 
 int
@@ -1788,27 +1817,52 @@ current_cu_count()
     return n;
 }
 
-int
-balanced_z_depth(int nx, int ny, int nz, int tile_x, int tile_y, int blocks_per_cu)
+// Blocks of the FP32 ring march over a region of nx x ny x nz cells: 64 x 8 (512 threads, one block
+// per CU) or 16 x 16 (two per CU). Both hold 512 cells per CU. The wide block reads fewer halo cells
+// and whole cache lines, and its two waves per SIMD cannot drift apart in z, which is what counts
+// once the fields outgrow the caches: at 512^3 16 x 16 blocks move 24 GB of HBM traffic per launch
+// (their neighbours' halo lines have left L2 when they come to them) and take 4.4 ms, 64 x 8 ones
+// 14 GB and 3.6 ms; 256^3 0.528 / 0.474 ms, 192 x 160 x 128 127 / 118 us, 128^3 58.1 / 56.9 us. Below
+// that the narrow block's finer grain is worth more (96^3 31.0 / 37.8 us), and so it is
+// where 64 x 8 tiles cover much more than the region.
+static bool
+ring_wide_blocks(int nx, int ny, int nz)
 {
-    // A z-march block costs its depth plus the 6 planes that fill its queues before the first
-    // output. Blocks are dispatched in rounds of `slots` (the resident block slots of the GPU),
-    // so a launch costs about rounds x (depth + 6). Splits of the box into k equal z-chunks of at
-    // least 8 planes are considered up to four times the k that fills every slot in the first
-    // round, and the cheapest is taken (the smallest k among equals). Equal chunks keep each
-    // XCD's contiguous block range equally loaded: an uneven last chunk leaves the XCDs that hold
-    // its blocks idle for the rest of the launch.
-    const long cols  = (long)((nx + tile_x - 1) / tile_x) * ((ny + tile_y - 1) / tile_y);
-    const long slots = (long)blocks_per_cu * current_cu_count();
-    const long kfill = std::max(1L, (slots + cols - 1) / cols);
-    const int kmax   = (int)std::max(1L, std::min(4 * kfill, (long)nz / 8));
-    int best_zd      = nz;
-    double best_cost = INFINITY;
+    if (AC_DOUBLE_PRECISION)
+        return false;
+    auto up          = [](long n, long t) { return (n + t - 1) / t * t; };
+    const long wide  = up(nx, 64) * up(ny, 8);
+    const long tiles = up(nx, 16) * up(ny, 16);
+    return (long)nx * ny * nz >= 1L << 21 && wide * 20 <= tiles * 21;
+}
+
+// z-depth of equal z-chunks for the ring march over nx x ny x nz cells (0: whole columns). A block
+// costs its planes plus a prologue (six planes to stage, three to scatter) worth `pro` of them;
+// blocks run in rounds of the GPU's resident block slots, and a round that leaves every CU one block
+// of two runs its planes in `light` of the time. Measured (FP32, 16 x 16 blocks, us): 3.1 a plane + 5
+// with two blocks per CU, 2.15 a plane + 3 with one; 64 x 8 blocks 2.85 a plane + 6; FP64 3.4 a
+// plane + 9. Equal chunks keep each XCD's contiguous block range equally loaded.
+static int
+ring_z_depth(int nx, int ny, int nz)
+{
+    const bool wide   = ring_wide_blocks(nx, ny, nz);
+    const int tx      = wide ? 64 : 16, ty = wide ? 8 : 16;
+    const int per_cu  = wide || AC_DOUBLE_PRECISION ? 1 : 2;
+    const double pro  = AC_DOUBLE_PRECISION ? 2.7 : wide ? 2.1 : 1.6;
+    const double light = per_cu == 2 ? 0.69 : 1.0;
+    const long cus    = current_cu_count();
+    const long cols   = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+    const long slots  = per_cu * cus;
+    const long kfill  = std::max(1L, (slots + cols - 1) / cols);
+    const int kmax    = (int)std::min(std::max(12L, 4 * kfill), (long)nz);
+    int best_zd       = nz;
+    double best_cost  = INFINITY;
     for (int k = 1; k <= kmax; ++k) {
-        const int zd       = (nz + k - 1) / k;
-        const long blocks  = cols * ((nz + zd - 1) / zd);
-        const long rounds  = (blocks + slots - 1) / slots;
-        const double cost  = (double)rounds * (zd + 6);
+        const int zd      = (nz + k - 1) / k;
+        const long blocks = cols * ((nz + zd - 1) / zd);
+        const long full = blocks / slots, rest = blocks % slots;
+        const double cost =
+            (zd + pro) * ((double)full + (rest == 0 ? 0.0 : rest <= cus ? light : 1.0));
         if (cost < best_cost) {
             best_cost = cost;
             best_zd   = zd;
@@ -1820,17 +1874,12 @@ balanced_z_depth(int nx, int ny, int nz, int tile_x, int tile_y, int blocks_per_
 AcKernelConfig
 default_kernel_config(int nx, int ny, int nz)
 {
-    // Fastest at 512^3: the lean z-march on 16 x 16 tiles with a 4-slot ring, loading the
-    // previous stage first and deferring its stores; in FP32 compiled for two waves per SIMD with
-    // pinned LDS windows (variant 19: two blocks of 4 waves per CU, 64 KiB of LDS each), in FP64
-    // for one wave per SIMD (variant 8: its 128 KiB ring leaves room for one block per CU). The
-    // z extent of a block is cut into equal chunks when the tile columns alone leave resident
-    // block slots empty (balanced_z_depth).
+    // Fastest at every size measured: the ring march (solve_ring.h).
     AcKernelConfig c;
     c.variant = AC_DOUBLE_PRECISION ? 8 : 19;
     c.tile_x  = 16;
     c.tile_y  = 16;
-    c.z_depth = balanced_z_depth(nx, ny, nz, c.tile_x, c.tile_y, AC_DOUBLE_PRECISION ? 1 : 2);
+    c.z_depth = ring_z_depth(nx, ny, nz);
     return c;
 }
 
@@ -1839,17 +1888,9 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
 {
     if (a.end.x <= a.start.x || a.end.y <= a.start.y || a.end.z <= a.start.z)
         return hipSuccess;
-    if (a.wrap) { // ghost cells read at their periodic images (the WRAP build)
-        if (a.cin[0] != nullptr || !kernel_config_reads_images(c))
-            return hipErrorInvalidConfiguration;
-#if AC_DOUBLE_PRECISION == 1
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 1, false, 4, true, true, 7, false, true>,
-                                          a, c.z_depth, stream);
-#else
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, true, true, 7, true, true>,
-                                          a, c.z_depth, stream);
-#endif
-    }
+    // ghost cells read at their periodic images: only the ring march does
+    if (a.wrap && (a.cin[0] != nullptr || !kernel_config_reads_images(c)))
+        return hipErrorInvalidConfiguration;
     if (a.cin[0] != nullptr) {
         // compensated integration: the lean z-march in its default tile, z-depth from `c`
         const int zd = c.variant >= 1 ? c.z_depth : 0;
@@ -1938,9 +1979,18 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     if (c.variant == 17 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 5, true, true, 7, true>,
                                           a, c.z_depth, stream);
-    if (c.variant == 19 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, true, true, 7, true>,
-                                          a, c.z_depth, stream);
+    if (c.variant == 19 && c.tile_x == 16 && c.tile_y == 16) {
+        if (!fields_equally_spaced(a))
+            return hipErrorInvalidValue;
+        if (ring_wide_blocks(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z))
+            return launch_zmarch_grid<64, 8>(solve_ring<64, 8, 2, false>, a, c.z_depth, stream);
+        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 2, false>, a, c.z_depth, stream);
+    }
+    if (c.variant == 24 && c.tile_x == 64 && c.tile_y == 8) {
+        if (!fields_equally_spaced(a))
+            return hipErrorInvalidValue;
+        return launch_zmarch_grid<64, 8>(solve_ring<64, 8, 2, false>, a, c.z_depth, stream);
+    }
     if (c.variant == 22 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, true, false, 7, true>,
                                           a, c.z_depth, stream);
@@ -1950,9 +2000,17 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
             solve_zlean<16, 16, 2, false, 5, true, true, 7, true, false, true>, a, c.z_depth,
             stream);
 #endif
+#if AC_DOUBLE_PRECISION == 1
+    if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16) {
+        if (!fields_equally_spaced(a))
+            return hipErrorInvalidValue;
+        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 1, false>, a, c.z_depth, stream);
+    }
+#else
     if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 1, false, 4, true, true>, a,
                                           c.z_depth, stream);
+#endif
 #undef AC_DIRECT
 #undef AC_ZMARCH
 #undef AC_ZMARCH2

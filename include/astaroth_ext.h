@@ -48,9 +48,8 @@ AcResult acDeviceReduceNoAlloc(const Device device, const Stream stream, const R
  * the interior, swap}, the caller sequence of the reference's single-GPU node loop
  * (src/core/node.cc:729-806). With the default kernel configuration (FP32 variant 19, FP64
  * variant 8; 16 x 16 tiles), compensated integration off and n >= 3 on every axis, the substeps
- * can instead read the periodic images of the ghost cells directly and make no fill: always in
- * FP64, in FP32 below 384^3 cells (above, its image-reading build is slower than the fills it
- * saves); acDeviceAutoOptimize measures both forms and keeps the faster, and
+ * can instead read the periodic images of the ghost cells directly and make no fill: by default
+ * below 512^3 cells (above, reading them costs more than the fills it saves); acDeviceAutoOptimize measures both forms and keeps the faster, and
  * acDeviceSetReadPeriodicImages overrides the choice. The state ends in `in` without a final
  * fill, as in the reference: its ghost cells are to be filled before they are read. */
 AcResult acDeviceIntegrateStep(const Device device, const Stream stream, const AcReal dt);
@@ -84,13 +83,19 @@ AcResult acDeviceIntegrateStepGraph(const Device device, const Stream stream, co
  * variants 5, 6: the lean z-march with a cell-major LDS ring (FP32).
  * variant 7: the lean z-march with a 5-slot ring, one barrier per plane.
  * variants 8, 9: the lean z-march loading the previous stage first and storing each output
- *            plane one step later; 4 and 5 ring slots (variant 8 is the FP64 default).
+ *            plane one step later; 4 and 5 ring slots. In FP64 variant 8 is the ring march, the
+ *            default.
  * variants 10-12: two-waves-per-SIMD builds of the lean z-march on 16 x 16 tiles (10: deferred
  *            stores, 11: previous stage first, 12: both).
  * variant 13: variant 12 with an 8-plane loop, whose LDS ring slots are compile-time (FP32).
  * variant 16: variant 12 with the 5-slot ring (one barrier per plane).
- * variants 17, 19, 22: variants 16, 12 and 10 reading each field's LDS stencil window through
- *            one pinned base register (FP32; variant 19 is the FP32 default).
+ * variants 17, 22: variants 16 and 10 reading each field's LDS stencil window through one pinned
+ *            base register (FP32).
+ * variant 19: the ring march (FP32 default): cross derivatives half scattered and half gathered, one
+ *            barrier per plane. Over regions of 2^21 cells or more that 64 x 8 blocks cover without
+ *            much waste it runs in such blocks of 512 threads instead of 16 x 16 ones; the results
+ *            are the same bit for bit.
+ * variant 24: the ring march in 64 x 8 blocks over any region (FP32).
  * variant 23: variant 17 with each plane loaded straight into its ring slot by direct-to-LDS
  *            loads (no staging registers or LDS writes; FP32). */
 typedef struct {

@@ -1,0 +1,57 @@
+"""The ring march (variant 19 in FP32, 8 in FP64; variant 24: its 64 x 8 blocks) at the sizes where a
+tiled march can go wrong: boxes smaller than a tile, tile edges and remainders, columns cut into chunks
+of one plane and more. Every chunk depth, block shape and ghost form (filled, or read at their periodic
+images) computes the same bits, and those are the oracle's.
+"""
+import numpy as np
+import pyoracle
+import pytest
+
+from astaroth_amd import abi
+from astaroth_amd.api import HostMesh, Library, real_params_double
+from astaroth_amd.initial import mhd_fields
+
+pytestmark = pytest.mark.gpu
+
+DIMS = [(3, 3, 3), (16, 16, 3), (17, 15, 4), (33, 18, 5), (64, 8, 3), (65, 9, 7), (15, 33, 10)]
+DT = 1e-3
+
+
+@pytest.mark.parametrize("dims", DIMS, ids=lambda d: "%dx%dx%d" % d)
+@pytest.mark.parametrize("double", [False, True], ids=["fp32", "fp64"])
+def test_ring_march_forms(double, dims):
+    nx, ny, nz = dims
+    lib = Library(double)
+    info = lib.config(n=nx, ny=ny, nz=nz)
+    fields = mhd_fields(nx, ny, nz, np.float64, config_id=6)
+    variants = [(8, 16, 16)] if double else [(19, 16, 16), (24, 64, 8)]
+    results = {}
+    for variant in variants:
+        for depth in (0, 1, 2, 3, 5):
+            for images in (0, 1):
+                if images and (variant[0] == 24 or min(dims) < abi.NGHOST):
+                    continue
+                with lib.device_create(0, info, autotune=False) as dev:
+                    dev.set_kernel_config(*variant, depth)
+                    if variant[0] != 24:
+                        assert lib.dll.acDeviceSetReadPeriodicImages(dev.handle, images) == abi.AC_SUCCESS
+                    mesh = HostMesh(lib, info, [f.astype(lib.dtype) for f in fields])
+                    dev.load_mesh(mesh)
+                    for _ in range(2):
+                        dev.integrate_step(DT)
+                    out = mesh.copy()
+                    dev.store_mesh(out)
+                results[variant + (depth, images)] = [out.interior(q) for q in range(8)]
+    first = next(iter(results.values()))
+    for key, got in results.items():
+        for q in range(8):
+            assert np.array_equal(got[q], first[q]), (dims, key, q)
+    ref = [f.astype(lib.dtype).astype(np.float64) for f in fields]
+    pyoracle.integrate_steps_gpu_form(ref, real_params_double(info), DT, 2)
+    # 6 substeps, each of which rounds a value once and adds an increment whose sums of about 20 terms
+    # carry a few roundings more: 4 ulps of the field's largest value per substep
+    eps = np.finfo(lib.dtype).eps
+    for q in range(8):
+        want = ref[q][3:-3, 3:-3, 3:-3]
+        scale = max(np.abs(want).max(), np.abs(fields[q]).max())
+        assert np.abs(first[q].astype(np.float64) - want).max() <= 24 * eps * scale, (dims, q)
