@@ -640,7 +640,7 @@ solve_zmarch2(const SubstepArgs a, const int zdepth, const int ntx, const int nt
 // registers and no LDS writes. Each wave waits for its own loads (vmcnt 0) before the step's
 // barrier, so after it the whole plane is in LDS. In FP64 a round of 64 doubles is two such
 // loads, lane l fetching the low or high half (l & 1) of double l / 2 of its half-round.
-template <int TX, int TY, bool COMP = false, int NSLOT = 4, bool DEFER = false,
+template <int TX, int TY, int NSLOT = 4, bool DEFER = false,
           bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool WRAP = false,
           bool DMA = false>
 struct ZMarchLean {
@@ -866,16 +866,6 @@ struct ZMarchLean {
             for (int f = 0; f < NF; ++f)
                 prev[f] = ld(a.out[f] + oz, ow);
         }
-        // compensated integration: the rounding-error terms of the output cell, loaded with the
-        // previous stage so that their latency is hidden behind the step's arithmetic
-        AcReal cin[COMP ? NF : 1], cprev[COMP ? NF : 1];
-        if (COMP && OUT) {
-#pragma unroll
-            for (int f = 0; f < NF; ++f) {
-                cin[f]   = ld(a.cin[f] + oz, ow);
-                cprev[f] = a.rk.step > 0 ? ld(a.cout[f] + oz, ow) : AcReal(0);
-            }
-        }
         if (PREV_FIRST)
             issue_loads(st, p + AHEAD);
 
@@ -1005,10 +995,6 @@ struct ZMarchLean {
         AcReal rate[NF];
         mhd_rates_agg(g, P, rate);
         push_queue(st, ro); // qv[f][2] is now plane z
-        if (COMP) {
-            store_compensated(st, rate, prev, cin, cprev, oz, ow, z);
-            return;
-        }
         if (a.rk.step == 0) {
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
@@ -1027,41 +1013,6 @@ struct ZMarchLean {
         st.res_z = z < ze ? z : -1;
         if (!DEFER)
             flush(st);
-    }
-
-    // Compensated update: the state is the pair (u, c) with u + c carrying the rounding error
-    // of every previous update (u in `in`/`out`, c in `cin`/`cout`). The increment is formed
-    // from the pairs and added with an error-free two-sum (Knuth's TwoSum), whose error term
-    // becomes the new compensation:
-    //   s = 0: d = beta_dt F + c_in
-    //   s > 0: d = beta (ab ((u_in - u_prev) + (c_in - c_prev)) + dt F) + c_in
-    //   u_out + c_out = u_in + d exactly.
-    // The stencils read u only.
-    __device__ __forceinline__ void store_compensated(const State& st, const AcReal* rate,
-                                                      const AcReal* prev, const AcReal* cin,
-                                                      const AcReal* cprev, unsigned long oz,
-                                                      unsigned ow, int z) const
-    {
-        if (!(z < ze && active))
-            return;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            const AcReal u  = st.qv[f][2];
-            const AcReal ci = cin[f];
-            AcReal d;
-            if (a.rk.step == 0) {
-                d = a.rk.beta_dt * rate[f] + ci;
-            }
-            else {
-                const AcReal cp = cprev[f];
-                d = a.rk.beta * (a.rk.ab * ((u - prev[f]) + (ci - cp)) + a.rk.dt * rate[f]) + ci;
-            }
-            const AcReal sum = u + d;
-            const AcReal bb  = sum - u;
-            const AcReal err = (u - (sum - bb)) + (d - bb);
-            st_global(a.out[f] + oz, ow, sum);
-            st_global(a.cout[f] + oz, ow, err);
-        }
     }
 };
 
@@ -1459,15 +1410,15 @@ strip_tile(const int b, const int ntx, const int nty, int& btx, int& bty, int& b
 }
 
 // One z-march column: tile (btx, bty) of box `a`, output planes [zs, min(zs + zdepth, end.z)).
-template <int TX, int TY, bool COMP = false, int NSLOT = 4, bool DEFER = false,
+template <int TX, int TY, int NSLOT = 4, bool DEFER = false,
           bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool WRAP = false,
           bool DMA = false>
 __device__ __forceinline__ void
 zlean_column(const SubstepArgs& a,
-             typename ZMarchLean<TX, TY, COMP, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>::Shared& sh,
+             typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>::Shared& sh,
              const int btx, const int bty, const int zs, const int zdepth)
 {
-    typedef ZMarchLean<TX, TY, COMP, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA> K;
+    typedef ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA> K;
     K k(a, sh);
     const int tid = threadIdx.x;
     k.wave        = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1586,17 +1537,17 @@ zlean_column(const SubstepArgs& a,
         K::wait_vm(); // no load into the ring is left in flight when the block moves on or ends
 }
 
-template <int TX, int TY, int W, bool COMP = false, int NSLOT = 4, bool DEFER = false,
+template <int TX, int TY, int W, int NSLOT = 4, bool DEFER = false,
           bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool WRAP = false,
           bool DMA = false>
 __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W)))
 solve_zlean(const SubstepArgs a, const int zdepth, const int ntx, const int nty)
 {
     __shared__
-        typename ZMarchLean<TX, TY, COMP, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>::Shared sh;
+        typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>::Shared sh;
     int btx, bty, btz;
     strip_tile(xcd_remap((int)blockIdx.x, (int)gridDim.x), ntx, nty, btx, bty, btz);
-    zlean_column<TX, TY, COMP, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>(
+    zlean_column<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>(
         a, sh, btx, bty, a.start.z + btz * zdepth, zdepth);
 }
 
@@ -1615,14 +1566,14 @@ solve_zlean_batch(const SubstepArgs* __restrict__ boxes, const BatchItem* __rest
 {
     // periodic images read directly: the ensemble step fills no ghosts between its substeps
     __shared__
-        typename ZMarchLean<TX, TY, false, NSLOT, DEFER, PREV_FIRST, 7, WIN, true>::Shared sh;
+        typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, 7, WIN, true>::Shared sh;
     // Round r takes items [r G, (r + 1) G) (G = gridDim.x), each XCD a contiguous range of them
     // (xcd_remap): consecutive items are mostly neighbouring tile columns of one box, whose halo
     // lines are then shared in one L2.
     const int slot = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     for (int it = slot; it < nitems; it += gridDim.x) {
         const BatchItem w = items[it];
-        zlean_column<TX, TY, false, NSLOT, DEFER, PREV_FIRST, 7, WIN, true>(
+        zlean_column<TX, TY, NSLOT, DEFER, PREV_FIRST, 7, WIN, true>(
             boxes[w.box], sh, w.btx, w.bty, w.zs, w.zdepth);
     }
 }
@@ -1892,13 +1843,16 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     if (a.wrap && (a.cin[0] != nullptr || !kernel_config_reads_images(c)))
         return hipErrorInvalidConfiguration;
     if (a.cin[0] != nullptr) {
-        // compensated integration: the lean z-march in its default tile, z-depth from `c`
+        // compensated integration: the ring march with the two error terms, z-depth from `c`
+        if (!fields_equally_spaced(a))
+            return hipErrorInvalidValue;
         const int zd = c.variant >= 1 ? c.z_depth : 0;
 #if AC_DOUBLE_PRECISION == 0
-        return launch_zmarch_grid<32, 4>(solve_zlean<32, 4, 1, true, 4, false, true>, a, zd,
-                                         stream);
+        if (ring_wide_blocks(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z))
+            return launch_zmarch_grid<64, 8>(solve_ring<64, 8, 2, true>, a, zd, stream);
+        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 2, true>, a, zd, stream);
 #else
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 1, true>, a, zd, stream);
+        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 1, true>, a, zd, stream);
 #endif
     }
 #define AC_DIRECT(TX, TY)                                                                          \
@@ -1947,37 +1901,37 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     if (c.variant == 6 && c.tile_x == 32 && c.tile_y == 4)
         return launch_zmarch_grid<32, 4>(solve_zaos<32, 4, 2>, a, c.z_depth, stream);
     if (c.variant == 7 && c.tile_x == 32 && c.tile_y == 4)
-        return launch_zmarch_grid<32, 4>(solve_zlean<32, 4, 1, false, 5>, a, c.z_depth, stream);
+        return launch_zmarch_grid<32, 4>(solve_zlean<32, 4, 1, 5>, a, c.z_depth, stream);
     if (c.variant == 7 && c.tile_x == 16 && c.tile_y == 8)
-        return launch_zmarch_grid<16, 8>(solve_zlean<16, 8, 1, false, 5>, a, c.z_depth, stream);
+        return launch_zmarch_grid<16, 8>(solve_zlean<16, 8, 1, 5>, a, c.z_depth, stream);
     if (c.variant == 8 && c.tile_x == 32 && c.tile_y == 4)
-        return launch_zmarch_grid<32, 4>(solve_zlean<32, 4, 1, false, 4, true, true>, a, c.z_depth,
+        return launch_zmarch_grid<32, 4>(solve_zlean<32, 4, 1, 4, true, true>, a, c.z_depth,
                                          stream);
     if (c.variant == 9 && c.tile_x == 32 && c.tile_y == 4)
-        return launch_zmarch_grid<32, 4>(solve_zlean<32, 4, 1, false, 5, true, true>, a, c.z_depth,
+        return launch_zmarch_grid<32, 4>(solve_zlean<32, 4, 1, 5, true, true>, a, c.z_depth,
                                          stream);
     // two waves per SIMD (16 x 16 is the only tile whose 4-slot ring leaves room for two blocks)
     if (c.variant == 10 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, true, false>, a,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, true, false>, a,
                                           c.z_depth, stream);
     if (c.variant == 11 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, false, true>, a,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, false, true>, a,
                                           c.z_depth, stream);
     if (c.variant == 12 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, true, true>, a,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, true, true>, a,
                                           c.z_depth, stream);
     // 8-phase plane loop (compile-time ring slots)
     if (c.variant == 13 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, true, true, 8>, a,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, true, true, 8>, a,
                                           c.z_depth, stream);
     // 5-slot ring (one barrier per plane), two waves per SIMD: 80 KiB of LDS per block
     if (c.variant == 16 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 5, true, true>, a,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 5, true, true>, a,
                                           c.z_depth, stream);
     // pinned LDS windows (WIN) on the two-wave builds: 5-slot ring; 4-slot ring with deferred
     // stores and previous stage first; 4-slot ring with deferred stores
     if (c.variant == 17 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 5, true, true, 7, true>,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 5, true, true, 7, true>,
                                           a, c.z_depth, stream);
     if (c.variant == 19 && c.tile_x == 16 && c.tile_y == 16) {
         if (!fields_equally_spaced(a))
@@ -1992,12 +1946,12 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
         return launch_zmarch_grid<64, 8>(solve_ring<64, 8, 2, false>, a, c.z_depth, stream);
     }
     if (c.variant == 22 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, false, 4, true, false, 7, true>,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, true, false, 7, true>,
                                           a, c.z_depth, stream);
     // direct-to-LDS plane loads into a 5-slot ring, pinned LDS windows
     if (c.variant == 23 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(
-            solve_zlean<16, 16, 2, false, 5, true, true, 7, true, false, true>, a, c.z_depth,
+            solve_zlean<16, 16, 2, 5, true, true, 7, true, false, true>, a, c.z_depth,
             stream);
 #endif
 #if AC_DOUBLE_PRECISION == 1
@@ -2008,7 +1962,7 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     }
 #else
     if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 1, false, 4, true, true>, a,
+        return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 1, 4, true, true>, a,
                                           c.z_depth, stream);
 #endif
 #undef AC_DIRECT

@@ -576,7 +576,12 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             const AcReal u = st.cur[f];
-            if (COMP) { // see ZMarchLean::store_compensated
+            if (COMP) {
+                // The state is the pair (u, c), u + c carrying the rounding error of every update
+                // before (u in in / out, c in cin / cout). The increment is formed from the pairs,
+                //   d = beta (ab ((u_in - u_prev) + (c_in - c_prev)) + dt F) + c_in,
+                // and added with an error-free two-sum (Knuth's TwoSum), whose error term is the
+                // new compensation: u_out + c_out = u_in + d exactly. The stencils read u only.
                 const AcReal ci = st.cin[f];
                 const AcReal diff = (u - st.prev[f]) + (ci - st.cprev[f]);
                 const AcReal d    = mad(a.rk.beta, mad(a.rk.dt, rate[f], a.rk.ab * diff), ci);

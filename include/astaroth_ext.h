@@ -126,8 +126,8 @@ AcResult acDeviceTimestepCFL(const Device device, const Stream stream, double* d
  * a second buffer (two more buffer sets, allocated and zeroed here) and each substep adds its
  * increment with an error-free two-sum: u_out + c_out = u_in + d exactly, where d includes
  * c_in. The right-hand side still reads the rounded state only. Loads, sets and randomisations
- * of a field reset its compensation to zero. The substep then always uses the lean z-march in
- * its default tile. enable == 0 frees the buffers. */
+ * of a field reset its compensation to zero. The substep then always uses the ring march (the
+ * default), with the configuration's z_depth. enable == 0 frees the buffers. */
 AcResult acDeviceSetCompensatedIntegration(const Device device, const int enable);
 
 /* ---- Synthetic initial conditions ----

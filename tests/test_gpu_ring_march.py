@@ -55,3 +55,34 @@ def test_ring_march_forms(double, dims):
         want = ref[q][3:-3, 3:-3, 3:-3]
         scale = max(np.abs(want).max(), np.abs(fields[q]).max())
         assert np.abs(first[q].astype(np.float64) - want).max() <= 24 * eps * scale, (dims, q)
+
+
+@pytest.mark.parametrize("dims", [(3, 4, 5), (17, 15, 4), (65, 9, 7)], ids=lambda d: "%dx%dx%d" % d)
+@pytest.mark.parametrize("double", [False, True], ids=["fp32", "fp64"])
+def test_ring_march_compensated(double, dims):
+    """The compensated build: the same bits for every chunk depth, and the oracle's values (tolerance
+    as above; the compensation only takes rounding away)."""
+    nx, ny, nz = dims
+    lib = Library(double)
+    info = lib.config(n=nx, ny=ny, nz=nz)
+    fields = mhd_fields(nx, ny, nz, np.float64, config_id=6)
+    results = []
+    for depth in (0, 1, 3):
+        with lib.device_create(0, info, autotune=False) as dev:
+            dev.set_kernel_config(8 if double else 19, 16, 16, depth)
+            dev.set_compensated_integration(True)
+            mesh = HostMesh(lib, info, [f.astype(lib.dtype) for f in fields])
+            dev.load_mesh(mesh)
+            for _ in range(2):
+                dev.integrate_step(DT)
+            out = mesh.copy()
+            dev.store_mesh(out)
+        results.append([out.interior(q) for q in range(8)])
+    ref = [f.astype(lib.dtype).astype(np.float64) for f in fields]
+    pyoracle.integrate_steps_gpu_form(ref, real_params_double(info), DT, 2)
+    eps = np.finfo(lib.dtype).eps
+    for q in range(8):
+        want = ref[q][3:-3, 3:-3, 3:-3]
+        scale = max(np.abs(want).max(), np.abs(fields[q]).max())
+        assert np.array_equal(results[1][q], results[0][q]) and np.array_equal(results[2][q], results[0][q]), (dims, q)
+        assert np.abs(results[0][q].astype(np.float64) - want).max() <= 24 * eps * scale, (dims, q)
