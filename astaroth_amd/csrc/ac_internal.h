@@ -82,10 +82,10 @@ struct SubstepArgs {
     RK3Coeffs rk;
 };
 
-// One work item of the batched solve: tile column (btx, bty) of box `box`, output planes
-// [zs, zs + zdepth) clipped to the box.
+// One work item of the batched solve: tile column (btx, bty) of box `box` (< 0: none), output planes
+// [zs, zs + zdepth) clipped to the box. `tall`: the tile is 32 x 16, not 64 x 8 (512-thread blocks).
 struct BatchItem {
-    int box, btx, bty, zs, zdepth;
+    int box, btx, bty, zs, zdepth, tall;
 };
 
 PhysParams make_phys_params(const AcMeshInfo& info);
@@ -100,8 +100,9 @@ bool kernel_config_reads_images(const AcKernelConfig& config);
 // Whether a periodic step of an n_x x n_y x n_z box reads the images rather than filling the ghost
 // cells, before the autotuner has measured both (the measured choice for the default builds).
 bool default_reads_images(int nx, int ny, int nz);
-// Batched solve (persistent lean z-march over a work list): `boxes` and `items` are device
-// arrays; tile shapes 32x4, 16x8, 16x16.
+// Batched solve (persistent ring march over a work list): `boxes` and `items` are device
+// arrays; tile shapes 32x4, 16x8, 16x16. The launch of FP32 tiles 64x8 takes 32x16 ones too
+// (BatchItem::tall); it is the ensemble's own choice, not one of the selectable shapes.
 bool batch_tile_supported(int tile_x, int tile_y);
 // Blocks of the batched solve build for this tile that are resident at once on the current
 // device (occupancy per CU x CUs), or -1 on error.

@@ -5,9 +5,9 @@
 // fields of m_x m_y m_z cells, x fastest) and its own AcMeshInfo (grid spacing, viscosity, ...).
 // One RK3 substep is
 //   * one periodic-fill launch over the ghost shells of all boxes (a flat list of ghost cells),
-//   * one persistent solve launch (solve_zlean_batch) over a (box, tile column, z range) work
-//     list sorted by decreasing cost, dealt to the resident blocks in rounds of one item per
-//     block, each XCD taking a contiguous range of a round's items,
+//   * one persistent solve launch (solve_ring_batch) over a (box, tile column, z range) work
+//     list, dealt out beforehand: the items by decreasing cost, each to the resident block with
+//     the least work so far,
 // and a step ends with per-box FP64 diagnostics (max and sum of squares of |u| and |A|, max, min
 // and sum of squares of lnrho) in two launches. acEnsembleIntegrateStepGraph records the whole
 // step once per (dt, buffer parity) into a HIP graph and replays it.
@@ -19,6 +19,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <queue>
 #include <vector>
 
 using namespace ac;
@@ -216,12 +217,14 @@ struct ensemble_s {
     size_t base_bytes;
     hipStream_t stream;
     int parity; // number of swaps mod 2: set `parity` holds the current state
-    // batched solve: one tile shape per launch; the z-depth of a box's work items is that of its
-    // size class (its column length n_z) when the tuner set one, else z_depth (0: whole columns)
+    // batched solve: one tile shape per launch (see launch_shape for 16 x 16); the z-depth of a
+    // box's work items is that of its size class (its column length n_z) when the ensemble chose
+    // it, else z_depth (0: whole columns)
     int tile_x, tile_y, z_depth, nblocks;
     std::map<int, int> class_depth;
     BatchItem* d_items;
     int nitems;
+    int2 launch; // tile shape of the launch
     SubstepArgs* d_args[3][2]; // per (substep, parity), for dt_args
     AcReal dt_args;
     bool args_valid;
@@ -276,48 +279,180 @@ box_depth(const Ensemble e, int nz)
     return (zd <= 0 || zd >= nz) ? nz : zd;
 }
 
-AcResult
-build_items(Ensemble e)
+// Planes a work item costs besides its outputs: it stages six planes and scatters three of them.
+constexpr int PROLOGUE = 3;
+
+// Tiles of one box for a launch: their shape, and the time of a plane of one relative to the others.
+struct Tiling {
+    int tx, ty, tall, weight;
+};
+
+int
+tiles(int n, int t)
+{
+    return (n + t - 1) / t;
+}
+
+// Cost of a plane of the box in whole tiles.
+long
+plane_cost(const Tiling& t, int3 n)
+{
+    return (long)tiles(n.x, t.tx) * tiles(n.y, t.ty) * t.weight;
+}
+
+// 512-thread blocks (FP32) take 64 x 8 tiles, or 32 x 16 ones in a box where those cover enough
+// fewer cells beyond it. A plane of either, and two of 16 x 16 (as many cells), take 81, 92 and 100:
+// 32 boxes of 64^3 0.836 / 0.933 / 1.002 ms per step (0.11 of it fill and diagnostics), 8 of 128^3
+// 1.69 / 1.78 / 1.97 ms, 16 of 96^3 (64 x 8 tiles cover 128 of 96) 1.93 / 1.65 / 1.87 ms. The wide
+// tiles read fewer halo cells and fewer parts of cache lines, which is what bounds a full chip here.
+Tiling
+wide_tiling(int3 n)
+{
+    const Tiling flat{64, 8, 0, 81}, tall{32, 16, 1, 92};
+    return plane_cost(flat, n) <= plane_cost(tall, n) ? flat : tall;
+}
+
+constexpr Tiling NARROW{16, 16, 0, 50};
+
+// Tile shape of the launch. In FP32 a 16 x 16 configuration runs 512-thread blocks if their tiles
+// cost less over the whole ensemble (32 boxes of 48^3, which they cover with a third to spare, take
+// 0.494 ms per step in 16 x 16 tiles and 0.556 in 64 x 8).
+int2
+launch_shape(const Ensemble e)
+{
+    if (!AC_DOUBLE_PRECISION && e->tile_x == 16 && e->tile_y == 16) {
+        long wide = 0, narrow = 0;
+        for (const AcMeshInfo& i : e->info) {
+            const int3 n = dims_of(i);
+            wide += plane_cost(wide_tiling(n), n) * n.z;
+            narrow += plane_cost(NARROW, n) * n.z;
+        }
+        if (wide < narrow)
+            return make_int2(64, 8);
+    }
+    return make_int2(e->tile_x, e->tile_y);
+}
+
+Tiling
+box_tiling(int2 launch, int3 n)
+{
+    return launch.x == 64 ? wide_tiling(n) : Tiling{launch.x, launch.y, 0, 1};
+}
+
+struct Deal {
+    std::vector<BatchItem> items; // slot s has items s, s + slots, ..., up to an empty one
+    int slots;
+    long makespan; // cost of the slot with the most work
+};
+
+// Work items at the current tile shape and z-depths, dealt to `slots` blocks: by decreasing cost,
+// each to the block with the least work so far (the lowest numbered of equals, which keeps
+// neighbouring tile columns in neighbouring slots).
+Deal
+deal_items(const Ensemble e, int2 launch, int slots)
 {
     struct Item {
         BatchItem w;
         long cost;
     };
     std::vector<Item> items;
-    const int TX = e->tile_x, TY = e->tile_y;
     for (int b = 0; b < e->nboxes; ++b) {
-        const int3 n  = dims_of(e->info[b]);
-        const int zd = box_depth(e, n.z);
-        const int ntx = (n.x + TX - 1) / TX, nty = (n.y + TY - 1) / TY, ntz = (n.z + zd - 1) / zd;
-        for (int tz = 0; tz < ntz; ++tz) {
-            const int zs    = NGHOST + tz * zd;
-            const int depth = std::min(zd, n.z + NGHOST - zs);
-            // planes marched: 6 warm-up planes plus the outputs
-            const long cost = 6 + depth;
-            for (int ty = 0; ty < nty; ++ty)
-                for (int tx = 0; tx < ntx; ++tx)
-                    items.push_back({{b, tx, ty, zs, zd}, cost});
-        }
+        const int3 n   = dims_of(e->info[b]);
+        const Tiling t = box_tiling(launch, n);
+        const int zd   = box_depth(e, n.z);
+        for (int zs = 0; zs < n.z; zs += zd)
+            for (int ty = 0; ty < tiles(n.y, t.ty); ++ty)
+                for (int tx = 0; tx < tiles(n.x, t.tx); ++tx)
+                    items.push_back({{b, tx, ty, NGHOST + zs, zd, t.tall},
+                                     (long)(PROLOGUE + std::min(zd, n.z - zs)) * t.weight});
     }
     std::stable_sort(items.begin(), items.end(),
                      [](const Item& a, const Item& b) { return a.cost > b.cost; });
-    std::vector<BatchItem> w(items.size());
-    for (size_t i = 0; i < items.size(); ++i)
-        w[i] = items[i].w;
+    Deal d;
+    d.slots    = (int)std::min<size_t>(slots, items.size());
+    d.makespan = 0;
+    typedef std::pair<long, int> Load; // work so far, slot
+    std::priority_queue<Load, std::vector<Load>, std::greater<Load>> least;
+    for (int s = 0; s < d.slots; ++s)
+        least.push({0, s});
+    std::vector<int> rounds(d.slots, 0);
+    const BatchItem none{-1, 0, 0, 0, 0, 0};
+    for (const Item& i : items) {
+        const Load l = least.top();
+        least.pop();
+        const size_t at = (size_t)rounds[l.second]++ * d.slots + l.second;
+        if (at >= d.items.size())
+            d.items.resize((at / d.slots + 1) * d.slots, none);
+        d.items[at] = i.w;
+        d.makespan  = std::max(d.makespan, l.first + i.cost);
+        least.push({l.first + i.cost, l.second});
+    }
+    return d;
+}
+
+AcResult
+build_items(Ensemble e)
+{
+    AC_HIP_CHECK(hipSetDevice(e->id));
+    const int2 launch = launch_shape(e);
+    // the persistent grid: one block per resident block slot of the batched kernel
+    const int slots = batch_resident_blocks(launch.x, launch.y);
+    if (slots < 1)
+        return AC_FAILURE;
+    const Deal d = deal_items(e, launch, slots);
+    if (d.items.size() > 0x7fffffffUL)
+        return AC_FAILURE;
     if (e->d_items)
         AC_HIP_CHECK(hipFree(e->d_items));
     e->d_items = nullptr;
-    e->nitems  = (int)w.size();
-    if (!w.empty()) {
-        AC_HIP_CHECK(hipMalloc((void**)&e->d_items, w.size() * sizeof(BatchItem)));
-        AC_HIP_CHECK(hipMemcpy(e->d_items, w.data(), w.size() * sizeof(BatchItem),
-                               hipMemcpyHostToDevice));
+    AC_HIP_CHECK(hipMalloc((void**)&e->d_items, d.items.size() * sizeof(BatchItem)));
+    AC_HIP_CHECK(hipMemcpy(e->d_items, d.items.data(), d.items.size() * sizeof(BatchItem),
+                           hipMemcpyHostToDevice));
+    e->launch  = launch;
+    e->nitems  = (int)d.items.size();
+    e->nblocks = d.slots;
+    return AC_SUCCESS;
+}
+
+// Every box's columns in equal parts of at most `depth` planes.
+std::map<int, int>
+equal_parts(const Ensemble e, int depth)
+{
+    std::map<int, int> d;
+    for (const AcMeshInfo& i : e->info) {
+        const int nz = dims_of(i).z;
+        d[nz]        = tiles(nz, tiles(nz, depth));
     }
-    // the persistent grid: one block per resident block slot of the batched kernel
+    return d;
+}
+
+// z-depths by decreasing promise: the work of the busiest block after the dealing, for columns cut
+// at 2 to 128 planes and whole ones. Fewer, longer items save prologues; more, shorter ones fill the
+// chip and leave less of a tail.
+AcResult
+rank_depths(Ensemble e, std::vector<std::map<int, int>>* ranked)
+{
     AC_HIP_CHECK(hipSetDevice(e->id));
-    e->nblocks = batch_resident_blocks(TX, TY);
-    if (e->nblocks < 1)
+    const int2 launch = launch_shape(e);
+    const int slots   = batch_resident_blocks(launch.x, launch.y);
+    if (slots < 1)
         return AC_FAILURE;
+    std::vector<std::pair<long, std::map<int, int>>> all;
+    for (const int depth : {1 << 30, 128, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4, 2}) {
+        const std::map<int, int> cut = equal_parts(e, depth);
+        if (!all.empty() && cut == all.back().second)
+            continue;
+        e->class_depth = cut;
+        const Deal d   = deal_items(e, launch, slots);
+        all.push_back({d.makespan, cut});
+        if (d.items.size() > 32 * (size_t)slots)
+            break; // shorter items only cost more
+    }
+    std::stable_sort(all.begin(), all.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+    ranked->clear();
+    for (const auto& c : all)
+        ranked->push_back(c.second);
+    e->class_depth = ranked->front();
     return AC_SUCCESS;
 }
 
@@ -402,7 +537,7 @@ enqueue_step(Ensemble e, int par0)
     // fill; one fill after the last substep leaves every box's ghosts current.
     int par = par0;
     for (int s = 0; s < 3; ++s) {
-        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, e->d_args[s][par], e->d_items,
+        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, e->d_args[s][par], e->d_items,
                                           e->nitems, e->nblocks, e->stream));
         par = 1 - par;
     }
@@ -428,12 +563,12 @@ time_batch(Ensemble e, int warm, int samples)
     AC_HIP_CHECK(hipEventCreate(&t1));
     const SubstepArgs* args = e->d_args[0][e->parity];
     for (int i = 0; i < warm; ++i)
-        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, args, e->d_items, e->nitems,
+        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, args, e->d_items, e->nitems,
                                           e->nblocks, e->stream));
     float best = INFINITY;
     for (int i = 0; i < samples; ++i) {
         AC_HIP_CHECK(hipEventRecord(t0, e->stream));
-        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, args, e->d_items, e->nitems,
+        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, args, e->d_items, e->nitems,
                                           e->nblocks, e->stream));
         AC_HIP_CHECK(hipEventRecord(t1, e->stream));
         AC_HIP_CHECK(hipEventSynchronize(t1));
@@ -446,16 +581,11 @@ time_batch(Ensemble e, int warm, int samples)
     return best;
 }
 
-// Tuned choices per ensemble composition (device, box sizes in order), kept for the process.
-struct EnsembleTuning {
-    int tile_x, tile_y;
-    std::map<int, int> class_depth;
-};
-
-std::map<std::vector<int>, EnsembleTuning>&
+// Tuned z-depths per ensemble composition (device, box sizes in order), kept for the process.
+std::map<std::vector<int>, std::map<int, int>>&
 tuning_cache()
 {
-    static std::map<std::vector<int>, EnsembleTuning> cache;
+    static std::map<std::vector<int>, std::map<int, int>> cache;
     return cache;
 }
 
@@ -500,8 +630,8 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     for (auto& i : e->info)
         acHostUpdateBuiltinParams(&i);
     e->parity   = 0;
-    // 16 x 16 tiles and whole columns, the fastest measured on the 96-box workload, until the
-    // tuner (below) measures this composition
+    // 16 x 16 tiles (or the wide ones of launch_shape), the z-depths ranked first until the tuner
+    // (below) measures this composition
     e->tile_x   = 16;
     e->tile_y   = 16;
     e->z_depth  = 0;
@@ -577,10 +707,11 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     AC_HIP_CHECK(hipMalloc((void**)&e->d_results, (size_t)nboxes * NDIAG * sizeof(double)));
     AC_HIP_CHECK(hipMemset(e->d_results, 0, (size_t)nboxes * NDIAG * sizeof(double)));
     AC_HIP_CHECK(hipHostMalloc((void**)&e->h_results, (size_t)nboxes * NDIAG * sizeof(double)));
-    if (build_items(e) != AC_SUCCESS)
+    std::vector<std::map<int, int>> ranked;
+    if (rank_depths(e, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
         return AC_FAILURE;
-    // Tile shape and per-class z-depths measured on this composition, as Devices tune at
-    // creation; AC_AUTOTUNE=0 keeps the defaults.
+    // z-depths measured on this composition, as Devices tune at creation; AC_AUTOTUNE=0 keeps the
+    // first.
     const char* tune = getenv("AC_AUTOTUNE");
     if (!(tune && tune[0] == '0') && acEnsembleAutoOptimize(e) != AC_SUCCESS)
         return AC_FAILURE;
@@ -654,77 +785,39 @@ acEnsembleAutoOptimize(Ensemble e)
         std::lock_guard<std::mutex> lock(tuning_mutex());
         const auto it = tuning_cache().find(key);
         if (it != tuning_cache().end()) {
-            e->tile_x      = it->second.tile_x;
-            e->tile_y      = it->second.tile_y;
+            e->tile_x = e->tile_y = 16;
             e->z_depth     = 0;
-            e->class_depth = it->second.class_depth;
+            e->class_depth = it->second;
             return build_items(e);
         }
     }
     // the timed launches need argument arrays; any dt times the same
     if (!e->args_valid && build_args(e, AcReal(1e-3)) != AC_SUCCESS)
         return AC_FAILURE;
-    // 1. The launch's tile shape, every box in whole columns.
-    const int shapes[3][2] = {{16, 16}, {16, 8}, {32, 4}};
+    e->tile_x = e->tile_y = 16;
     e->z_depth = 0;
-    e->class_depth.clear();
-    float best = INFINITY;
-    int bx = 16, by = 16;
-    for (const auto& s : shapes) {
-        e->tile_x = s[0];
-        e->tile_y = s[1];
-        if (build_items(e) != AC_SUCCESS)
-            continue;
-        const float ms = time_batch(e, 2, 3);
-        if (ms < best) {
-            best = ms;
-            bx   = s[0];
-            by   = s[1];
-        }
-    }
-    e->tile_x = bx;
-    e->tile_y = by;
-    if (build_items(e) != AC_SUCCESS)
+    std::vector<std::map<int, int>> ranked;
+    if (rank_depths(e, &ranked) != AC_SUCCESS)
         return AC_FAILURE;
-    // 2. Per size class (the column length n_z), the class with the most cells first: whole
-    // columns, or columns cut into 2, 3 or 4 equal z ranges. A cut shortens the longest work
-    // items (the launch's tail) at the cost of 6 warm-up planes per extra item; it is kept only
-    // when the whole launch gets at least 2 % faster.
-    std::map<int, double> work;
-    for (const AcMeshInfo& i : e->info) {
-        const int3 n = dims_of(i);
-        work[n.z] += (double)n.x * n.y * n.z;
-    }
-    std::vector<std::pair<double, int>> classes;
-    for (const auto& kv : work)
-        classes.push_back({kv.second, kv.first});
-    std::sort(classes.rbegin(), classes.rend());
-    best = time_batch(e, 1, 3);
-    for (const auto& c : classes) {
-        const int nz = c.second;
-        int keep     = 0;
-        for (const int parts : {2, 3, 4}) {
-            const int d = (nz + parts - 1) / parts;
-            if (d < 8 || d >= nz)
-                continue;
-            e->class_depth[nz] = d;
+    ranked.resize(std::min<size_t>(ranked.size(), 4));
+    float best = INFINITY;
+    size_t keep = 0;
+    for (int round = 0; round < 2; ++round) // twice: the clocks still rise during the first
+        for (size_t i = 0; i < ranked.size(); ++i) {
+            e->class_depth = ranked[i];
             if (build_items(e) != AC_SUCCESS)
                 return AC_FAILURE;
-            const float ms = time_batch(e, 1, 3);
-            if (ms < 0.98f * best) {
+            const float ms = time_batch(e, 1, 2);
+            if (round > 0 && ms < best) {
                 best = ms;
-                keep = d;
+                keep = i;
             }
         }
-        if (keep > 0)
-            e->class_depth[nz] = keep;
-        else
-            e->class_depth.erase(nz);
-        if (build_items(e) != AC_SUCCESS)
-            return AC_FAILURE;
-    }
+    e->class_depth = ranked[keep];
+    if (build_items(e) != AC_SUCCESS)
+        return AC_FAILURE;
     std::lock_guard<std::mutex> lock(tuning_mutex());
-    tuning_cache()[key] = EnsembleTuning{e->tile_x, e->tile_y, e->class_depth};
+    tuning_cache()[key] = e->class_depth;
     return AC_SUCCESS;
 }
 

@@ -631,9 +631,6 @@ solve_zmarch2(const SubstepArgs a, const int zdepth, const int ntx, const int nt
 // WIN: every stencil read of one field in one ring plane goes through one LDS base register
 // (the window's first cell, pinned in a VGPR), so that all its reads pair into ds_read2 with
 // immediate offsets; otherwise the compiler forms a new base (one VALU add) for most pairs.
-// WRAP: the tile halos and the planes above and below the box are read at their periodic images
-// inside the interior, so no ghost cell is read and the ghosts need not be filled first (the
-// values read are the same as after a periodic fill).
 // DMA (5-slot ring only): plane p + 1 is loaded straight into its ring slot with direct-to-LDS
 // loads (global_load_lds_dword: lane l of a wave writes the 4 bytes it loads to the wave's LDS
 // base + 4 l), issued at the start of step p into the slot that plane p - 4 left; no staging
@@ -641,8 +638,7 @@ solve_zmarch2(const SubstepArgs a, const int zdepth, const int ntx, const int nt
 // barrier, so after it the whole plane is in LDS. In FP64 a round of 64 doubles is two such
 // loads, lane l fetching the low or high half (l & 1) of double l / 2 of its half-round.
 template <int TX, int TY, int NSLOT = 4, bool DEFER = false,
-          bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool WRAP = false,
-          bool DMA = false>
+          bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool DMA = false>
 struct ZMarchLean {
     static_assert(NQ == 7 || (NQ == 8 && NSLOT == 4), "8-phase loop needs the 4-slot ring");
     static_assert(!DMA || NSLOT == 5, "direct-to-LDS staging needs the 5-slot ring");
@@ -729,12 +725,7 @@ struct ZMarchLean {
 
     __device__ __forceinline__ void issue_loads(State& st, int p) const
     {
-        int q = min(p, zmax);
-        if (WRAP) { // periodic image of a ghost plane (planes run 0 .. zmax = nz + 5)
-            const int nz = zmax - 5;
-            q = q < NGHOST ? q + nz : q >= nz + NGHOST ? q - nz : q;
-        }
-        const long pl = (long)q * a.mxy;
+        const long pl = (long)min(p, zmax) * a.mxy;
         unsigned go[R][NH];
 #pragma unroll
         for (int r = 0; r < R; ++r)
@@ -1411,14 +1402,13 @@ strip_tile(const int b, const int ntx, const int nty, int& btx, int& bty, int& b
 
 // One z-march column: tile (btx, bty) of box `a`, output planes [zs, min(zs + zdepth, end.z)).
 template <int TX, int TY, int NSLOT = 4, bool DEFER = false,
-          bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool WRAP = false,
-          bool DMA = false>
+          bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool DMA = false>
 __device__ __forceinline__ void
 zlean_column(const SubstepArgs& a,
-             typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>::Shared& sh,
+             typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, DMA>::Shared& sh,
              const int btx, const int bty, const int zs, const int zdepth)
 {
-    typedef ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA> K;
+    typedef ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, DMA> K;
     K k(a, sh);
     const int tid = threadIdx.x;
     k.wave        = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1439,13 +1429,8 @@ zlean_column(const SubstepArgs& a,
             const int e  = K::NH == 1 ? tid + r * K::NT
                                       : r * K::NT + (tid & ~63) + h * 32 + ((tid & 63) >> 1);
             const int ex = e % K::LX, ey = e / K::LX;
-            int xx = x0 - 3 + ex, yy = y0 - 3 + ey;
+            const int xx = x0 - 3 + ex, yy = y0 - 3 + ey;
             const bool in_box = e < K::LN && xx < a.mx && yy < a.my;
-            if (WRAP) { // periodic images of the x and y ghost columns
-                const int nx = a.mx - 2 * NGHOST, ny = a.my - 2 * NGHOST;
-                xx = xx < NGHOST ? xx + nx : xx >= nx + NGHOST ? xx - nx : xx;
-                yy = yy < NGHOST ? yy + ny : yy >= ny + NGHOST ? yy - ny : yy;
-            }
             k.goff[r][h] = (unsigned)(in_box ? xx + yy * a.mx : 0) * sizeof(AcReal) +
                            (K::NH == 1 ? 0u : (unsigned)(tid & 1) * 4u);
         }
@@ -1538,51 +1523,17 @@ zlean_column(const SubstepArgs& a,
 }
 
 template <int TX, int TY, int W, int NSLOT = 4, bool DEFER = false,
-          bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool WRAP = false,
-          bool DMA = false>
+          bool PREV_FIRST = false, int NQ = 7, bool WIN = false, bool DMA = false>
 __global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W)))
 solve_zlean(const SubstepArgs a, const int zdepth, const int ntx, const int nty)
 {
     __shared__
-        typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>::Shared sh;
+        typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, DMA>::Shared sh;
     int btx, bty, btz;
     strip_tile(xcd_remap((int)blockIdx.x, (int)gridDim.x), ntx, nty, btx, bty, btz);
-    zlean_column<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, WRAP, DMA>(
+    zlean_column<TX, TY, NSLOT, DEFER, PREV_FIRST, NQ, WIN, DMA>(
         a, sh, btx, bty, a.start.z + btz * zdepth, zdepth);
 }
-
-// Persistent form for ensembles of independent boxes: a grid sized to the resident block slots
-// walks a (box, tile column, z range) work list; each box brings its own arguments (pointers,
-// sizes, physical parameters), read from global memory.
-// The 16 x 16 FP32 build has the single-box default's options (4-slot ring, previous stage
-// first, deferred stores, pinned LDS windows, two waves per SIMD): 7.93 ms per 96-box step
-// against 8.87 ms for a 5-slot ring without pinned windows, which spills 20 registers to
-// scratch (interleaved on one box, work items dealt to XCDs in contiguous ranges).
-template <int TX, int TY, int W = 1, int NSLOT = 4, bool DEFER = false, bool PREV_FIRST = false,
-          bool WIN = false>
-__global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W)))
-solve_zlean_batch(const SubstepArgs* __restrict__ boxes, const BatchItem* __restrict__ items,
-                  const int nitems)
-{
-    // periodic images read directly: the ensemble step fills no ghosts between its substeps
-    __shared__
-        typename ZMarchLean<TX, TY, NSLOT, DEFER, PREV_FIRST, 7, WIN, true>::Shared sh;
-    // Round r takes items [r G, (r + 1) G) (G = gridDim.x), each XCD a contiguous range of them
-    // (xcd_remap): consecutive items are mostly neighbouring tile columns of one box, whose halo
-    // lines are then shared in one L2.
-    const int slot = xcd_remap((int)blockIdx.x, (int)gridDim.x);
-    for (int it = slot; it < nitems; it += gridDim.x) {
-        const BatchItem w = items[it];
-        zlean_column<TX, TY, NSLOT, DEFER, PREV_FIRST, 7, WIN, true>(
-            boxes[w.box], sh, w.btx, w.bty, w.zs, w.zdepth);
-    }
-}
-
-#if AC_DOUBLE_PRECISION == 0
-#define AC_BATCH16 solve_zlean_batch<16, 16, 2, 4, true, true, true>
-#else
-#define AC_BATCH16 solve_zlean_batch<16, 16>
-#endif
 
 // ------------------------------------------------------------------------------------------
 // configuration table
@@ -1691,6 +1642,57 @@ solve_ring(const SubstepArgs a, const int zdepth, const int ntx, const int nty)
     strip_tile(xcd_remap((int)blockIdx.x, (int)gridDim.x), ntx, nty, btx, bty, btz);
     ring_column<TX, TY, COMP>(a, sh, btx, bty, a.start.z + btz * zdepth, zdepth);
 }
+
+// Persistent form for ensembles of independent boxes: a grid sized to the resident block slots
+// walks a (box, tile column, z range) work list; each box brings its own arguments (pointers,
+// sizes, physical parameters), read from global memory. Periodic images are read directly
+// (SubstepArgs::wrap): the ensemble step fills no ghosts between its substeps.
+// Each item's arguments are copied: left in memory, the plane loop loads them again (62 scalar loads
+// a plane, which share their counter with the LDS reads; 200 boxes of 32^3 in FP32 1009 -> 982 us per
+// step, 96 boxes in FP64 16.47 -> 16.26 ms).
+//
+// Slot s takes items s, s + G, s + 2 G, ... (G = gridDim.x) up to its first empty one (box < 0);
+// slots are numbered so that each XCD has a contiguous range (xcd_remap): neighbouring slots mostly
+// hold neighbouring tile columns of one box, whose halo lines are then shared in one L2.
+template <int TX, int TY, int W>
+__global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W)))
+solve_ring_batch(const SubstepArgs* __restrict__ boxes, const BatchItem* __restrict__ items,
+                 const int nitems)
+{
+    __shared__ typename ZMarchRing<TX, TY, false>::Shared sh;
+    for (int it = xcd_remap((int)blockIdx.x, (int)gridDim.x); it < nitems; it += gridDim.x) {
+        const BatchItem w = items[it];
+        if (w.box < 0)
+            break;
+        const SubstepArgs a = boxes[w.box];
+        ring_column<TX, TY, false>(a, sh, w.btx, w.bty, w.zs, w.zdepth);
+    }
+}
+
+#if AC_DOUBLE_PRECISION == 0
+// The same with 512-thread blocks, each box in 64 x 8 or 32 x 16 tiles (BatchItem::tall).
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+solve_ring_batch_wide(const SubstepArgs* __restrict__ boxes, const BatchItem* __restrict__ items,
+                      const int nitems)
+{
+    __shared__ union {
+        ZMarchRing<64, 8, false>::Shared flat;
+        ZMarchRing<32, 16, false>::Shared tall;
+    } sh;
+    for (int it = xcd_remap((int)blockIdx.x, (int)gridDim.x); it < nitems; it += gridDim.x) {
+        const BatchItem w = items[it];
+        if (w.box < 0)
+            break;
+        const SubstepArgs a = boxes[w.box];
+        if (w.tall)
+            ring_column<32, 16, false>(a, sh.tall, w.btx, w.bty, w.zs, w.zdepth);
+        else
+            ring_column<64, 8, false>(a, sh.flat, w.btx, w.bty, w.zs, w.zdepth);
+    }
+}
+#endif
+
+constexpr int BATCH_WAVES = sizeof(AcReal) == 4 ? 2 : 1; // waves per SIMD, as the single-box builds
 
 } // namespace
 
@@ -1951,7 +1953,7 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     // direct-to-LDS plane loads into a 5-slot ring, pinned LDS windows
     if (c.variant == 23 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(
-            solve_zlean<16, 16, 2, 5, true, true, 7, true, false, true>, a, c.z_depth,
+            solve_zlean<16, 16, 2, 5, true, true, 7, true, true>, a, c.z_depth,
             stream);
 #endif
 #if AC_DOUBLE_PRECISION == 1
@@ -1977,41 +1979,45 @@ batch_tile_supported(int tx, int ty)
     return (tx == 32 && ty == 4) || (tx == 16 && ty == 8) || (tx == 16 && ty == 16);
 }
 
+typedef void (*BatchKernel)(const SubstepArgs*, const BatchItem*, int);
+
+static BatchKernel
+batch_kernel(int tx, int ty)
+{
+#if AC_DOUBLE_PRECISION == 0
+    if (tx == 64 && ty == 8)
+        return solve_ring_batch_wide;
+#endif
+    if (tx == 32 && ty == 4)
+        return solve_ring_batch<32, 4, BATCH_WAVES>;
+    if (tx == 16 && ty == 8)
+        return solve_ring_batch<16, 8, BATCH_WAVES>;
+    if (tx == 16 && ty == 16)
+        return solve_ring_batch<16, 16, BATCH_WAVES>;
+    return nullptr;
+}
+
 hipError_t
 launch_substep_batch(int tx, int ty, const SubstepArgs* boxes, const BatchItem* items, int nitems,
                      int nblocks, hipStream_t stream)
 {
-    if (nitems <= 0)
-        return hipSuccess;
-    if (nblocks <= 0 || nblocks > nitems)
-        nblocks = nitems;
-    if (tx == 32 && ty == 4)
-        solve_zlean_batch<32, 4><<<dim3(nblocks), dim3(128), 0, stream>>>(boxes, items, nitems);
-    else if (tx == 16 && ty == 8)
-        solve_zlean_batch<16, 8><<<dim3(nblocks), dim3(128), 0, stream>>>(boxes, items, nitems);
-    else if (tx == 16 && ty == 16)
-        AC_BATCH16<<<dim3(nblocks), dim3(256), 0, stream>>>(boxes, items, nitems);
-    else
+    const BatchKernel kernel = batch_kernel(tx, ty);
+    if (!kernel || nblocks <= 0 || nitems <= 0)
         return hipErrorInvalidConfiguration;
+    kernel<<<dim3(nblocks), dim3(tx * ty), 0, stream>>>(boxes, items, nitems);
     return hipGetLastError();
 }
 
 int
 batch_resident_blocks(int tx, int ty)
 {
+    const BatchKernel kernel = batch_kernel(tx, ty);
     int per_cu = 0, cus = 0, dev = 0;
-    hipError_t e = hipErrorInvalidConfiguration;
-    if (tx == 32 && ty == 4)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, solve_zlean_batch<32, 4>, 128, 0);
-    else if (tx == 16 && ty == 8)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, solve_zlean_batch<16, 8>, 128, 0);
-    else if (tx == 16 && ty == 16)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, AC_BATCH16, 256, 0);
-    if (e != hipSuccess || hipGetDevice(&dev) != hipSuccess ||
+    if (!kernel || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tx * ty, 0) != hipSuccess ||
+        hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return -1;
     return per_cu * cus;
 }
-#undef AC_BATCH16
 
 } // namespace ac

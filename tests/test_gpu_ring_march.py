@@ -86,3 +86,31 @@ def test_ring_march_compensated(double, dims):
         scale = max(np.abs(want).max(), np.abs(fields[q]).max())
         assert np.array_equal(results[1][q], results[0][q]) and np.array_equal(results[2][q], results[0][q]), (dims, q)
         assert np.abs(results[0][q].astype(np.float64) - want).max() <= 24 * eps * scale, (dims, q)
+
+
+@pytest.mark.parametrize("dims", [((64, 8, 5), (128, 9, 7), (32, 16, 40), (33, 17, 12), (3, 4, 5)), ((48, 48, 9), (17, 15, 4))],
+                         ids=["wide", "narrow"])
+@pytest.mark.parametrize("double", [False, True], ids=["fp32", "fp64"])
+def test_ring_march_batched(double, dims):
+    """Boxes at the edges of the batched launch's tile shapes: the same bits as box after box (the
+    march writes out every multiply-add, so a cell's value depends on no tile or z range)."""
+    lib = Library(double)
+    infos = [lib.config(n=nx, ny=ny, nz=nz, AC_nu_visc=1e-3 * (b + 1)) for b, (nx, ny, nz) in enumerate(dims)]
+    out = {}
+    for mode, depth in (("looped", None), ("batched", None), ("batched", 0), ("graph", 3)):
+        with lib.ensemble_create(infos) as ens:
+            if depth is not None:
+                ens.set_kernel_config(16, 16, depth)
+            for b, d in enumerate(dims):
+                ens.load_mesh(b, HostMesh(lib, infos[b], [f.astype(lib.dtype) for f in mhd_fields(*d, np.float64, config_id=4)]))
+            for _ in range(2):
+                ens.integrate_step(DT, mode=mode)
+            for b in range(len(dims)):
+                mesh = HostMesh(lib, infos[b])
+                ens.store_mesh(b, mesh)
+                out.setdefault(b, []).append([mesh.interior(q).copy() for q in range(8)])
+    for b, d in enumerate(dims):
+        for q in range(8):
+            assert np.abs(out[b][0][q]).max() > 0, (d, q)
+            for other in out[b][1:]:
+                assert np.array_equal(other[q], out[b][0][q]), (d, q)
