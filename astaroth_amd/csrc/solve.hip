@@ -1009,7 +1009,11 @@ struct ZMarchLean {
 
 } // namespace
 } // namespace ac
+#if AC_DOUBLE_PRECISION == 0
 #include "solve_ring.h"
+#else
+#include "solve_pair.h"
+#endif
 namespace ac {
 namespace {
 
@@ -1597,7 +1601,7 @@ typedef void (*ZMarchKernel)(const SubstepArgs, const int, const int, const int)
 
 template <int TX, int TY>
 hipError_t
-launch_zmarch_grid(ZMarchKernel kernel, const SubstepArgs& a, int zdepth, hipStream_t stream)
+launch_zmarch_grid(ZMarchKernel kernel, const SubstepArgs& a, int zdepth, hipStream_t stream, int threads = TX * TY)
 {
     const int nx = a.end.x - a.start.x, ny = a.end.y - a.start.y, nz = a.end.z - a.start.z;
     const int ntx = (nx + TX - 1) / TX, nty = (ny + TY - 1) / TY;
@@ -1607,7 +1611,7 @@ launch_zmarch_grid(ZMarchKernel kernel, const SubstepArgs& a, int zdepth, hipStr
     const long nblocks = (long)ntx * nty * ntz;
     if (nblocks > 0x7fffffffL)
         return hipErrorInvalidConfiguration;
-    kernel<<<dim3((unsigned)nblocks), dim3(TX * TY), 0, stream>>>(a, zdepth, ntx, nty);
+    kernel<<<dim3((unsigned)nblocks), dim3(threads), 0, stream>>>(a, zdepth, ntx, nty);
     return hipGetLastError();
 }
 
@@ -1633,14 +1637,24 @@ launch_direct(const SubstepArgs& a, hipStream_t stream)
 }
 
 
-template <int TX, int TY, int W, bool COMP>
-__global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W)))
+// Two waves per SIMD in both precisions (FP64 blocks have two threads per cell column).
+template <int TX, int TY, bool COMP>
+__global__ void __launch_bounds__((RingColumn<TX, TY, COMP>::NT)) __attribute__((amdgpu_waves_per_eu(2)))
 solve_ring(const SubstepArgs a, const int zdepth, const int ntx, const int nty)
 {
-    __shared__ typename ZMarchRing<TX, TY, COMP>::Shared sh;
+    __shared__ typename RingColumn<TX, TY, COMP>::Shared sh;
     int btx, bty, btz;
     strip_tile(xcd_remap((int)blockIdx.x, (int)gridDim.x), ntx, nty, btx, bty, btz);
     ring_column<TX, TY, COMP>(a, sh, btx, bty, a.start.z + btz * zdepth, zdepth);
+}
+
+template <int TX, int TY, bool COMP>
+hipError_t
+launch_ring(const SubstepArgs& a, int zdepth, hipStream_t stream)
+{
+    if (!fields_equally_spaced(a))
+        return hipErrorInvalidValue;
+    return launch_zmarch_grid<TX, TY>(solve_ring<TX, TY, COMP>, a, zdepth, stream, RingColumn<TX, TY, COMP>::NT);
 }
 
 // Persistent form for ensembles of independent boxes: a grid sized to the resident block slots
@@ -1654,12 +1668,12 @@ solve_ring(const SubstepArgs a, const int zdepth, const int ntx, const int nty)
 // Slot s takes items s, s + G, s + 2 G, ... (G = gridDim.x) up to its first empty one (box < 0);
 // slots are numbered so that each XCD has a contiguous range (xcd_remap): neighbouring slots mostly
 // hold neighbouring tile columns of one box, whose halo lines are then shared in one L2.
-template <int TX, int TY, int W>
-__global__ void __launch_bounds__(TX* TY) __attribute__((amdgpu_waves_per_eu(W)))
+template <int TX, int TY>
+__global__ void __launch_bounds__((RingColumn<TX, TY, false>::NT)) __attribute__((amdgpu_waves_per_eu(2)))
 solve_ring_batch(const SubstepArgs* __restrict__ boxes, const BatchItem* __restrict__ items,
                  const int nitems)
 {
-    __shared__ typename ZMarchRing<TX, TY, false>::Shared sh;
+    __shared__ typename RingColumn<TX, TY, false>::Shared sh;
     for (int it = xcd_remap((int)blockIdx.x, (int)gridDim.x); it < nitems; it += gridDim.x) {
         const BatchItem w = items[it];
         if (w.box < 0)
@@ -1676,8 +1690,8 @@ solve_ring_batch_wide(const SubstepArgs* __restrict__ boxes, const BatchItem* __
                       const int nitems)
 {
     __shared__ union {
-        ZMarchRing<64, 8, false>::Shared flat;
-        ZMarchRing<32, 16, false>::Shared tall;
+        RingColumn<64, 8, false>::Shared flat;
+        RingColumn<32, 16, false>::Shared tall;
     } sh;
     for (int it = xcd_remap((int)blockIdx.x, (int)gridDim.x); it < nitems; it += gridDim.x) {
         const BatchItem w = items[it];
@@ -1692,7 +1706,6 @@ solve_ring_batch_wide(const SubstepArgs* __restrict__ boxes, const BatchItem* __
 }
 #endif
 
-constexpr int BATCH_WAVES = sizeof(AcReal) == 4 ? 2 : 1; // waves per SIMD, as the single-box builds
 
 } // namespace
 
@@ -1793,15 +1806,15 @@ ring_wide_blocks(int nx, int ny, int nz)
 // costs its planes plus a prologue (six planes to stage, three to scatter) worth `pro` of them;
 // blocks run in rounds of the GPU's resident block slots, and a round that leaves every CU one block
 // of two runs its planes in `light` of the time. Measured (FP32, 16 x 16 blocks, us): 3.1 a plane + 5
-// with two blocks per CU, 2.15 a plane + 3 with one; 64 x 8 blocks 2.85 a plane + 6; FP64 3.4 a
-// plane + 9. Equal chunks keep each XCD's contiguous block range equally loaded.
+// with two blocks per CU, 2.15 a plane + 3 with one; 64 x 8 blocks 2.85 a plane + 6; FP64 2.5 a
+// plane + 8. Equal chunks keep each XCD's contiguous block range equally loaded.
 static int
 ring_z_depth(int nx, int ny, int nz)
 {
     const bool wide   = ring_wide_blocks(nx, ny, nz);
     const int tx      = wide ? 64 : 16, ty = wide ? 8 : 16;
     const int per_cu  = wide || AC_DOUBLE_PRECISION ? 1 : 2;
-    const double pro  = AC_DOUBLE_PRECISION ? 2.7 : wide ? 2.1 : 1.6;
+    const double pro  = AC_DOUBLE_PRECISION ? 3.3 : wide ? 2.1 : 1.6;
     const double light = per_cu == 2 ? 0.69 : 1.0;
     const long cus    = current_cu_count();
     const long cols   = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
@@ -1846,16 +1859,12 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
         return hipErrorInvalidConfiguration;
     if (a.cin[0] != nullptr) {
         // compensated integration: the ring march with the two error terms, z-depth from `c`
-        if (!fields_equally_spaced(a))
-            return hipErrorInvalidValue;
         const int zd = c.variant >= 1 ? c.z_depth : 0;
 #if AC_DOUBLE_PRECISION == 0
         if (ring_wide_blocks(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z))
-            return launch_zmarch_grid<64, 8>(solve_ring<64, 8, 2, true>, a, zd, stream);
-        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 2, true>, a, zd, stream);
-#else
-        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 1, true>, a, zd, stream);
+            return launch_ring<64, 8, true>(a, zd, stream);
 #endif
+        return launch_ring<16, 16, true>(a, zd, stream);
     }
 #define AC_DIRECT(TX, TY)                                                                          \
     if (c.variant == 0 && c.tile_x == TX && c.tile_y == TY)                                        \
@@ -1936,16 +1945,12 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 5, true, true, 7, true>,
                                           a, c.z_depth, stream);
     if (c.variant == 19 && c.tile_x == 16 && c.tile_y == 16) {
-        if (!fields_equally_spaced(a))
-            return hipErrorInvalidValue;
         if (ring_wide_blocks(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z))
-            return launch_zmarch_grid<64, 8>(solve_ring<64, 8, 2, false>, a, c.z_depth, stream);
-        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 2, false>, a, c.z_depth, stream);
+            return launch_ring<64, 8, false>(a, c.z_depth, stream);
+        return launch_ring<16, 16, false>(a, c.z_depth, stream);
     }
     if (c.variant == 24 && c.tile_x == 64 && c.tile_y == 8) {
-        if (!fields_equally_spaced(a))
-            return hipErrorInvalidValue;
-        return launch_zmarch_grid<64, 8>(solve_ring<64, 8, 2, false>, a, c.z_depth, stream);
+        return launch_ring<64, 8, false>(a, c.z_depth, stream);
     }
     if (c.variant == 22 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, true, false, 7, true>,
@@ -1958,9 +1963,7 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
 #endif
 #if AC_DOUBLE_PRECISION == 1
     if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16) {
-        if (!fields_equally_spaced(a))
-            return hipErrorInvalidValue;
-        return launch_zmarch_grid<16, 16>(solve_ring<16, 16, 1, false>, a, c.z_depth, stream);
+        return launch_ring<16, 16, false>(a, c.z_depth, stream);
     }
 #else
     if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16)
@@ -1989,12 +1992,18 @@ batch_kernel(int tx, int ty)
         return solve_ring_batch_wide;
 #endif
     if (tx == 32 && ty == 4)
-        return solve_ring_batch<32, 4, BATCH_WAVES>;
+        return solve_ring_batch<32, 4>;
     if (tx == 16 && ty == 8)
-        return solve_ring_batch<16, 8, BATCH_WAVES>;
+        return solve_ring_batch<16, 8>;
     if (tx == 16 && ty == 16)
-        return solve_ring_batch<16, 16, BATCH_WAVES>;
+        return solve_ring_batch<16, 16>;
     return nullptr;
+}
+
+static int
+batch_threads(int tx, int ty)
+{
+    return tx * ty * (RingColumn<16, 16, false>::NT / 256);
 }
 
 hipError_t
@@ -2004,7 +2013,7 @@ launch_substep_batch(int tx, int ty, const SubstepArgs* boxes, const BatchItem* 
     const BatchKernel kernel = batch_kernel(tx, ty);
     if (!kernel || nblocks <= 0 || nitems <= 0)
         return hipErrorInvalidConfiguration;
-    kernel<<<dim3(nblocks), dim3(tx * ty), 0, stream>>>(boxes, items, nitems);
+    kernel<<<dim3(nblocks), dim3(batch_threads(tx, ty)), 0, stream>>>(boxes, items, nitems);
     return hipGetLastError();
 }
 
@@ -2013,7 +2022,7 @@ batch_resident_blocks(int tx, int ty)
 {
     const BatchKernel kernel = batch_kernel(tx, ty);
     int per_cu = 0, cus = 0, dev = 0;
-    if (!kernel || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tx * ty, 0) != hipSuccess ||
+    if (!kernel || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, batch_threads(tx, ty), 0) != hipSuccess ||
         hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return -1;

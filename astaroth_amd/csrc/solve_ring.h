@@ -1,4 +1,5 @@
-// The ring march: the default solve of both precisions (variant 19 in FP32, 8 in FP64).
+// The ring march: the default FP32 solve (variant 19). FP64 runs it with two threads per cell column
+// (solve_pair.h).
 //
 // A block owns a TX x TY column of cells and marches it along z, one thread per cell column, all
 // eight fields of four planes in an LDS ring. What it does differently from the lean z-march
@@ -22,16 +23,14 @@
 //   serves every field's x window, and rows a tile row apart start 16 banks apart (16-wide tiles).
 // * The previous stage is loaded a whole plane ahead, the next plane too.
 // * One field pointer and a stride instead of sixteen pointers, which in this march spilled 78 scalar
-//   registers to lanes of vector ones (50 v_readlane a plane in FP32; FP64 100 -> 77). The rates are
+//   registers to lanes of vector ones (50 v_readlane a plane). The rates are
 //   formed with fewer operations (mhd_rates_lean). The vector instruction count is level with the
 //   lean march's (630 a plane in FP32): what it gains is in the waits.
 //
-// What bounds it: in FP32 the vector pipes are busy 65 % of the time on boxes that fit the caches (LDS
-// 50 %); at 512^3 the launch moves 14 GB, 85 % of what a plain copy reaches on this card. In FP64 one
-// 256-thread block per CU (its ring takes 121 KiB of the 160) leaves LDS and memory latency exposed
-// between its barriers. Per launch, sustained (us): FP32 32^3 27.9 -> 7.8, 97 x 61 x 75 35.8 -> 26.2,
-// 128^3 74.7 -> 57.9, 256^3 529 -> 456, 512^3 4020 -> 3600; FP64 64^3 47 -> 26.7, 128^3 173 -> 140,
-// 256^3 1265 -> 1020, 512^3 9900 -> 8160.
+// What bounds it: the vector pipes are busy 65 to 73 % of the time on boxes that fit the caches (LDS
+// 50 %); at 512^3 the launch moves 14 GB, 85 % of what a plain copy reaches on this card. Per launch,
+// sustained (us), lean march -> this: 32^3 27.9 -> 7.8, 97 x 61 x 75 35.8 -> 26.2, 128^3 74.7 -> 57.9,
+// 256^3 529 -> 456, 512^3 4020 -> 3600.
 #pragma once
 #include "physics.h"
 
@@ -89,22 +88,10 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
     static __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
     // Values that are to be computed here: nothing else keeps the compiler from putting off a
     // field's arithmetic, with its whole window in registers, to where the results are used (up to
-    // 470 spilled registers). Settling less leaves it more freedom to order the rest; FP64 runs
-    // fastest with the cross sums settled (256^3 1.02 ms against 1.10), FP32 with the derivatives
-    // (3.58 ms at 512^3 against 3.65 with both).
-    static constexpr bool SETTLE_SUMS = sizeof(AcReal) == 8 && !COMP;
+    // 470 spilled registers). The derivatives are settled, the cross sums are not, which leaves it
+    // freedom to order the rest (3.58 ms at 512^3 against 3.65 with both).
     static __device__ __forceinline__ void settle_one(AcReal& v) { asm volatile("" : "+v"(v)); }
-    template <typename... T> static __device__ __forceinline__ void settle_now(T&... v) { (settle_one(v), ...); }
-    template <typename... T> static __device__ __forceinline__ void settle(T&... v)
-    {
-        if constexpr (!SETTLE_SUMS)
-            settle_now(v...);
-    }
-    template <typename... T> static __device__ __forceinline__ void settle_sums(T&... v)
-    {
-        if constexpr (SETTLE_SUMS)
-            settle_now(v...);
-    }
+    template <typename... T> static __device__ __forceinline__ void settle(T&... v) { (settle_one(v), ...); }
     static __device__ __forceinline__ unsigned pin(unsigned off)
     {
         asm volatile("" : "+v"(off));
@@ -255,7 +242,6 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
             st.x[n][PH] = mad(-c[3], d[2], st.x[n][PH]);
         else
             st.x[n][PH] = -(c[3] * d[2]);
-        settle_sums(st.x[n][0], st.x[n][1], st.x[n][2]);
     }
 
     __device__ __forceinline__ Rows rows(int slot) const
@@ -320,7 +306,6 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
         sum[1] = mad(cy, h.yz[1] - h.yz[0], sum[1]);
         sum[2] = mad(cx, h.xx[1] - h.xx[0], sum[2]);
         sum[2] = mad(cy, h.yy[1] - h.yy[0], sum[2]);
-        settle_sums(sum[0], sum[1], sum[2]);
     }
 
     // In-plane part of output plane z (ring slot PH; planes z+1, z+2 in the next two slots). The LDS
@@ -530,7 +515,7 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
             g.ug[2][2]   = first(l, d1z);
             g.ulap[2] += st.own[2];
         }
-        settle_now(g.lr_z, g.lr_lap, g.ug[0][2], g.ulap[0], g.ug[1][2], g.ulap[1], g.ug[2][2], g.ulap[2], st.own[2]);
+        settle(g.lr_z, g.lr_lap, g.ug[0][2], g.ulap[0], g.ug[1][2], g.ulap[1], g.ug[2][2], g.ulap[2], st.own[2]);
         fence();
         const LdsReal *rm = row(st.s3, -3), *rp = row(st.s3, 3);
         const Ahead u3 = ahead<3>(r3, rm, rp, VTXBUF_UUX), a3 = ahead<3>(r3, rm, rp, VTXBUF_AX);
@@ -557,7 +542,7 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
             g.s_z        = first(l, d1z);
             g.s_lap += second(l, st.cur[VTXBUF_ENTROPY], d2z);
         }
-        settle_now(g.alap[0], st.rest[0], g.B[1], g.alap[1], st.rest[1], g.B[0], g.alap[2], g.s_z, g.s_lap);
+        settle(g.alap[0], st.rest[0], g.B[1], g.alap[1], st.rest[1], g.B[0], g.alap[2], g.s_z, g.s_lap);
         fence();
         w  = rows(st.s1);
         lr = star(w, VTXBUF_LNRHO);
@@ -666,6 +651,8 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
         }
     }
 };
+
+template <int TX, int TY, bool COMP> using RingColumn = ZMarchRing<TX, TY, COMP>;
 
 // One z-march column: tile (btx, bty) of box `a`, output planes [zs, min(zs + zdepth, end.z)).
 template <int TX, int TY, bool COMP>
