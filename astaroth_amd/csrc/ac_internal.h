@@ -171,11 +171,9 @@ struct device_s {
     long field_stride;     // cells from one field of a set to the next
     double* reduce_partials;
     double* reduce_scratch; // this GPU's copy of the library's reduction scratch array
-    double* reduce_result;
-    double* reduce_result_host; // pinned
+    double* reduce_result; // pinned host memory
     double* diag_partials;      // acDeviceDiagnostics: per-block partials, results, pinned copy
-    double* diag_result;
-    double* diag_result_host;
+    double* diag_result; // pinned host memory
     AcKernelConfig kernel_config;
     // periodic steps read the ghost cells' images where the configuration has such a build
     // (default by size, measured by acDeviceAutoOptimize, set by acDeviceSetReadPeriodicImages)

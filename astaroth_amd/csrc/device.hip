@@ -203,10 +203,8 @@ reduce_impl(const Device d, Stream stream, ReductionType rtype, int nvals, const
     hipStream_t s = d->streams[stream];
     AC_HIP_CHECK(launch_reduce((int)rtype, nvals, vals, d->local_config, d->reduce_partials,
                                reduce_partials_needed(), d->reduce_result, s));
-    AC_HIP_CHECK(hipMemcpyAsync(d->reduce_result_host, d->reduce_result, sizeof(double),
-                                hipMemcpyDeviceToHost, s));
     AC_HIP_CHECK(hipStreamSynchronize(s));
-    *result = *d->reduce_result_host;
+    *result = *d->reduce_result;
     return AC_SUCCESS;
 }
 
@@ -512,11 +510,11 @@ acDeviceCreate(const int id, const AcMeshInfo config, Device* device_handle)
         d->base_in[q] = d->vba.in[q];
     }
     AC_HIP_CHECK(hipMalloc((void**)&d->reduce_partials, sizeof(double) * reduce_partials_needed()));
-    AC_HIP_CHECK(hipMalloc((void**)&d->reduce_result, sizeof(double)));
-    AC_HIP_CHECK(hipHostMalloc((void**)&d->reduce_result_host, sizeof(double), hipHostMallocDefault));
+    // in host memory, where the last kernel of a reduction writes its result: a copy there from
+    // device memory is a kernel of its own (3.4 us and a gap; 128^3 steps with a time step and diagnostics each 244 -> 240 us)
+    AC_HIP_CHECK(hipHostMalloc((void**)&d->reduce_result, sizeof(double), hipHostMallocDefault));
     AC_HIP_CHECK(hipMalloc((void**)&d->diag_partials, sizeof(double) * diagnostics_partials_needed()));
-    AC_HIP_CHECK(hipMalloc((void**)&d->diag_result, 9 * sizeof(double)));
-    AC_HIP_CHECK(hipHostMalloc((void**)&d->diag_result_host, 9 * sizeof(double), hipHostMallocDefault));
+    AC_HIP_CHECK(hipHostMalloc((void**)&d->diag_result, 9 * sizeof(double), hipHostMallocDefault));
     AC_HIP_CHECK(hipStreamSynchronize(d->streams[0]));
     // this GPU's copy of the reduction scratch array (acDeviceReduceNoAlloc), with `id` current
     AC_HIP_CHECK(reduce_scratch_address(id, &d->reduce_scratch));
@@ -542,11 +540,9 @@ acDeviceDestroy(Device device)
     for (int set = 0; set < 2; ++set)
         AC_HIP_CHECK(hipFree(device->field_sets[set]));
     AC_HIP_CHECK(hipFree(device->reduce_partials));
-    AC_HIP_CHECK(hipFree(device->reduce_result));
-    AC_HIP_CHECK(hipHostFree(device->reduce_result_host));
+    AC_HIP_CHECK(hipHostFree(device->reduce_result));
     AC_HIP_CHECK(hipFree(device->diag_partials));
-    AC_HIP_CHECK(hipFree(device->diag_result));
-    AC_HIP_CHECK(hipHostFree(device->diag_result_host));
+    AC_HIP_CHECK(hipHostFree(device->diag_result));
     if (device->halo_buffer)
         AC_HIP_CHECK(hipFree(device->halo_buffer));
     for (int set = 0; set < 2; ++set)
@@ -1468,12 +1464,10 @@ acDeviceDiagnostics(const Device device, const Stream stream, double* out)
         f[q] = device->vba.in[q];
     AC_HIP_CHECK(launch_diagnostics(f, device->local_config, device->diag_partials,
                                     device->diag_result, s));
-    AC_HIP_CHECK(hipMemcpyAsync(device->diag_result_host, device->diag_result, 9 * sizeof(double),
-                                hipMemcpyDeviceToHost, s));
     AC_HIP_CHECK(hipStreamSynchronize(s));
     const double n = (double)nx_of(device) * ny_of(device) * nz_of(device);
     for (int i = 0; i < 9; ++i)
-        out[i] = i % 3 == 2 ? std::sqrt(device->diag_result_host[i] / n) : device->diag_result_host[i];
+        out[i] = i % 3 == 2 ? std::sqrt(device->diag_result[i] / n) : device->diag_result[i];
     return AC_SUCCESS;
 }
 
