@@ -1783,23 +1783,29 @@ current_cu_count()
     return n;
 }
 
-// Blocks of the FP32 ring march over a region of nx x ny x nz cells: 64 x 8 (512 threads, one block
-// per CU) or 16 x 16 (two per CU). Both hold 512 cells per CU. The wide block reads fewer halo cells
-// and whole cache lines, and its two waves per SIMD cannot drift apart in z, which is what counts
-// once the fields outgrow the caches: at 512^3 16 x 16 blocks move 24 GB of HBM traffic per launch
-// (their neighbours' halo lines have left L2 when they come to them) and take 4.4 ms, 64 x 8 ones
-// 14 GB and 3.6 ms; 256^3 0.528 / 0.474 ms, 192 x 160 x 128 127 / 118 us, 128^3 58.1 / 56.9 us. Below
-// that the narrow block's finer grain is worth more (96^3 31.0 / 37.8 us), and so it is
-// where 64 x 8 tiles cover much more than the region.
-static bool
-ring_wide_blocks(int nx, int ny, int nz)
+// Tile of the ring march over a region of nx x ny x nz cells. FP32 chooses between 64 x 8 and 32 x 16 (512
+// threads, one block per CU) and 16 x 16 (two per CU): all hold 512 cells per CU. The wide blocks read
+// fewer halo cells and parts of cache lines, and their two waves per SIMD cannot drift apart in z,
+// which is what counts once the fields outgrow the caches: at 512^3 16 x 16 blocks move 24 GB of HBM
+// traffic per launch (their neighbours' halo lines have left L2 when they come to them) and take
+// 4.4 ms, 64 x 8 ones 14 GB and 3.58 ms, 32 x 16 ones 3.68; 256^3 0.528 / 0.474 ms, 192 x 160 x 128 127 /
+// 118 us, 128^3 58.1 / 56.9 us. Below that the narrow block's finer grain is worth more (96^3 31.0 / 37.8
+// us, 32 x 16 33.6). Above, the tiles that cover the region at the least cost: 16 x 16 against 32 x 16
+// 352^3 1619 / 1255 us, 224^3 402 / 356, 160^3 137 / 126, 416 x 96 x 96 126 / 118.
+static int2
+ring_tile(int nx, int ny, int nz)
 {
-    if (AC_DOUBLE_PRECISION)
-        return false;
-    auto up          = [](long n, long t) { return (n + t - 1) / t * t; };
-    const long wide  = up(nx, 64) * up(ny, 8);
-    const long tiles = up(nx, 16) * up(ny, 16);
-    return (long)nx * ny * nz >= 1L << 21 && wide * 20 <= tiles * 21;
+    const int2 tile[3] = {make_int2(16, 16), make_int2(64, 8), make_int2(32, 16)};
+    const long cost[3] = {112, 100, 103}; // per cell of the tiles, relative
+    int best           = 0;
+    if (!AC_DOUBLE_PRECISION && (long)nx * ny * nz >= 1L << 21) {
+        auto up = [](long n, long t) { return (n + t - 1) / t * t; };
+        auto of = [&](int i) { return up(nx, tile[i].x) * up(ny, tile[i].y) * cost[i]; };
+        for (int i = 1; i < 3; ++i)
+            if (of(i) < of(best))
+                best = i;
+    }
+    return tile[best];
 }
 
 // z-depth of equal z-chunks for the ring march over nx x ny x nz cells (0: whole columns). A block
@@ -1811,8 +1817,9 @@ ring_wide_blocks(int nx, int ny, int nz)
 static int
 ring_z_depth(int nx, int ny, int nz)
 {
-    const bool wide   = ring_wide_blocks(nx, ny, nz);
-    const int tx      = wide ? 64 : 16, ty = wide ? 8 : 16;
+    const int2 tile   = ring_tile(nx, ny, nz);
+    const int tx      = tile.x, ty = tile.y;
+    const bool wide   = tx * ty == 512;
     const int per_cu  = wide || AC_DOUBLE_PRECISION ? 1 : 2;
     const double pro  = AC_DOUBLE_PRECISION ? 3.3 : wide ? 2.1 : 1.6;
     const double light = per_cu == 2 ? 0.69 : 1.0;
@@ -1849,6 +1856,20 @@ default_kernel_config(int nx, int ny, int nz)
     return c;
 }
 
+template <bool COMP>
+static hipError_t
+launch_ring_tile(const SubstepArgs& a, int zdepth, hipStream_t stream)
+{
+#if AC_DOUBLE_PRECISION == 0
+    const int2 tile = ring_tile(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z);
+    if (tile.x == 64)
+        return launch_ring<64, 8, COMP>(a, zdepth, stream);
+    if (tile.x == 32)
+        return launch_ring<32, 16, COMP>(a, zdepth, stream);
+#endif
+    return launch_ring<16, 16, COMP>(a, zdepth, stream);
+}
+
 hipError_t
 launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream)
 {
@@ -1860,11 +1881,7 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     if (a.cin[0] != nullptr) {
         // compensated integration: the ring march with the two error terms, z-depth from `c`
         const int zd = c.variant >= 1 ? c.z_depth : 0;
-#if AC_DOUBLE_PRECISION == 0
-        if (ring_wide_blocks(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z))
-            return launch_ring<64, 8, true>(a, zd, stream);
-#endif
-        return launch_ring<16, 16, true>(a, zd, stream);
+        return launch_ring_tile<true>(a, zd, stream);
     }
 #define AC_DIRECT(TX, TY)                                                                          \
     if (c.variant == 0 && c.tile_x == TX && c.tile_y == TY)                                        \
@@ -1944,14 +1961,10 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     if (c.variant == 17 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 5, true, true, 7, true>,
                                           a, c.z_depth, stream);
-    if (c.variant == 19 && c.tile_x == 16 && c.tile_y == 16) {
-        if (ring_wide_blocks(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z))
-            return launch_ring<64, 8, false>(a, c.z_depth, stream);
-        return launch_ring<16, 16, false>(a, c.z_depth, stream);
-    }
-    if (c.variant == 24 && c.tile_x == 64 && c.tile_y == 8) {
+    if (c.variant == 19 && c.tile_x == 16 && c.tile_y == 16)
+        return launch_ring_tile<false>(a, c.z_depth, stream);
+    if (c.variant == 24 && c.tile_x == 64 && c.tile_y == 8)
         return launch_ring<64, 8, false>(a, c.z_depth, stream);
-    }
     if (c.variant == 22 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, true, false, 7, true>,
                                           a, c.z_depth, stream);
@@ -1962,9 +1975,8 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
             stream);
 #endif
 #if AC_DOUBLE_PRECISION == 1
-    if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16) {
-        return launch_ring<16, 16, false>(a, c.z_depth, stream);
-    }
+    if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16)
+        return launch_ring_tile<false>(a, c.z_depth, stream);
 #else
     if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 1, 4, true, true>, a,

@@ -92,9 +92,9 @@ AcResult acDeviceIntegrateStepGraph(const Device device, const Stream stream, co
  * variants 17, 22: variants 16 and 10 reading each field's LDS stencil window through one pinned
  *            base register (FP32).
  * variant 19: the ring march (FP32 default): cross derivatives half scattered and half gathered, one
- *            barrier per plane. Over regions of 2^21 cells or more that 64 x 8 blocks cover without
- *            much waste it runs in such blocks of 512 threads instead of 16 x 16 ones; the results
- *            are the same bit for bit.
+ *            barrier per plane. Over regions of 2^21 cells or more that 64 x 8 or 32 x 16 blocks
+ *            cover without much waste it runs in such blocks of 512 threads instead of 16 x 16
+ *            ones; the results are the same bit for bit.
  * variant 24: the ring march in 64 x 8 blocks over any region (FP32).
  * variant 23: variant 17 with each plane loaded straight into its ring slot by direct-to-LDS
  *            loads (no staging registers or LDS writes; FP32). */

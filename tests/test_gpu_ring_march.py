@@ -114,3 +114,28 @@ def test_ring_march_batched(double, dims):
             assert np.abs(out[b][0][q]).max() > 0, (d, q)
             for other in out[b][1:]:
                 assert np.array_equal(other[q], out[b][0][q]), (d, q)
+
+
+@pytest.mark.parametrize("dims", [(352, 96, 63), (350, 90, 70), (450, 49, 97)], ids=lambda d: "%dx%dx%d" % d)
+def test_ring_march_tiles(dims):
+    """FP32 regions of 2^21 cells or more, whose tile goes by what covers them: the same bits as in
+    64 x 8 tiles, with and without compensation."""
+    nx, ny, nz = dims
+    assert nx * ny * nz >= 2**21
+    lib = Library(False)
+    info = lib.config(n=nx, ny=ny, nz=nz)
+    for compensated in (False, True):
+        out = []
+        for config in ((19, 16, 16, 0), (19, 16, 16, 11), (24, 64, 8, 0)):
+            with lib.device_create(0, info, autotune=False) as dev:
+                dev.set_kernel_config(*config)
+                dev.set_compensated_integration(compensated)
+                for q in range(8):
+                    dev.randomize_uniform(q, -1e-3, 1e-3, 7 * q + 1)
+                dev.integrate_step(DT)
+                mesh = HostMesh(lib, info)
+                dev.store_mesh(mesh)
+                out.append([mesh.interior(q).copy() for q in range(8)])
+        for q in range(8):
+            assert np.abs(out[0][q]).max() > 0
+            assert np.array_equal(out[1][q], out[0][q]) and np.array_equal(out[2][q], out[0][q]), (dims, compensated, q)
