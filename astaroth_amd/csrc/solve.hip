@@ -1737,8 +1737,9 @@ default_reads_images(int nx, int ny, int nz)
     // (the far-side halo and plane reads). Per step, images against fills (ms, sustained):
     //   FP32  128^3 0.176 / 0.201   256^3 1.45 / 1.47   384^3 4.93 / 5.04   448^3 7.91 / 8.06
     //         512^3 11.80 / 11.40
-    //   FP64  128^3 0.406 / 0.458   256^3 3.08 / 3.20   384^3 10.85 / 11.04   512^3 25.07 / 25.16
-    // so images below 512^3 cells.
+    //   FP64  128^3 0.351 / 0.400   256^3 2.65 / 2.79   384^3 9.40 / 9.71   512^3 21.6 / 22.1
+    // so images below 512^3 cells, in FP64 too: its crossover lies higher, but a caller of a 512^3 box
+    // has found its ghosts filled by the step.
     return (double)nx * ny * nz < 512.0 * 512.0 * 512.0;
 }
 

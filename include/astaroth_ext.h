@@ -83,8 +83,8 @@ AcResult acDeviceIntegrateStepGraph(const Device device, const Stream stream, co
  * variants 5, 6: the lean z-march with a cell-major LDS ring (FP32).
  * variant 7: the lean z-march with a 5-slot ring, one barrier per plane.
  * variants 8, 9: the lean z-march loading the previous stage first and storing each output
- *            plane one step later; 4 and 5 ring slots. In FP64 variant 8 is the ring march, the
- *            default.
+ *            plane one step later; 4 and 5 ring slots. In FP64 variant 8 is the ring march with
+ *            two threads per cell column, the default.
  * variants 10-12: two-waves-per-SIMD builds of the lean z-march on 16 x 16 tiles (10: deferred
  *            stores, 11: previous stage first, 12: both).
  * variant 13: variant 12 with an 8-plane loop, whose LDS ring slots are compile-time (FP32).
