@@ -1784,41 +1784,19 @@ current_cu_count()
     return n;
 }
 
-// Tile of the ring march over a region of nx x ny x nz cells. FP32 chooses between 64 x 8 and 32 x 16 (512
-// threads, one block per CU) and 16 x 16 (two per CU): all hold 512 cells per CU. The wide blocks read
-// fewer halo cells and parts of cache lines, and their two waves per SIMD cannot drift apart in z,
-// which is what counts once the fields outgrow the caches: at 512^3 16 x 16 blocks move 24 GB of HBM
-// traffic per launch (their neighbours' halo lines have left L2 when they come to them) and take
-// 4.4 ms, 64 x 8 ones 14 GB and 3.58 ms, 32 x 16 ones 3.68; 256^3 0.528 / 0.474 ms, 192 x 160 x 128 127 /
-// 118 us, 128^3 58.1 / 56.9 us. Below that the narrow block's finer grain is worth more (96^3 31.0 / 37.8
-// us, 32 x 16 33.6). Above, the tiles that cover the region at the least cost: 16 x 16 against 32 x 16
-// 352^3 1619 / 1255 us, 224^3 402 / 356, 160^3 137 / 126, 416 x 96 x 96 126 / 118.
-static int2
-ring_tile(int nx, int ny, int nz)
-{
-    const int2 tile[3] = {make_int2(16, 16), make_int2(64, 8), make_int2(32, 16)};
-    const long cost[3] = {112, 100, 103}; // per cell of the tiles, relative
-    int best           = 0;
-    if (!AC_DOUBLE_PRECISION && (long)nx * ny * nz >= 1L << 21) {
-        auto up = [](long n, long t) { return (n + t - 1) / t * t; };
-        auto of = [&](int i) { return up(nx, tile[i].x) * up(ny, tile[i].y) * cost[i]; };
-        for (int i = 1; i < 3; ++i)
-            if (of(i) < of(best))
-                best = i;
-    }
-    return tile[best];
-}
-
-// z-depth of equal z-chunks for the ring march over nx x ny x nz cells (0: whole columns). A block
+// Equal z-chunks for the ring march over nx x ny x nz cells in `tile`: their depth and the cost. A block
 // costs its planes plus a prologue (six planes to stage, three to scatter) worth `pro` of them;
 // blocks run in rounds of the GPU's resident block slots, and a round that leaves every CU one block
 // of two runs its planes in `light` of the time. Measured (FP32, 16 x 16 blocks, us): 3.1 a plane + 5
 // with two blocks per CU, 2.15 a plane + 3 with one; 64 x 8 blocks 2.85 a plane + 6; FP64 2.5 a
 // plane + 8. Equal chunks keep each XCD's contiguous block range equally loaded.
-static int
-ring_z_depth(int nx, int ny, int nz)
+struct RingPlan {
+    int zdepth;
+    double cost; // planes of one block
+};
+static RingPlan
+ring_plan(int2 tile, int nx, int ny, int nz)
 {
-    const int2 tile   = ring_tile(nx, ny, nz);
     const int tx      = tile.x, ty = tile.y;
     const bool wide   = tx * ty == 512;
     const int per_cu  = wide || AC_DOUBLE_PRECISION ? 1 : 2;
@@ -1842,7 +1820,47 @@ ring_z_depth(int nx, int ny, int nz)
             best_zd   = zd;
         }
     }
-    return best_zd >= nz ? 0 : best_zd;
+    return {best_zd, best_cost};
+}
+
+// Tile of the ring march over a region of nx x ny x nz cells. FP32 chooses between 64 x 8 and 32 x 16 (512
+// threads, one block per CU) and 16 x 16 (two per CU): all hold 512 cells per CU. The wide blocks read
+// fewer halo cells and parts of cache lines, and their two waves per SIMD cannot drift apart in z,
+// which is what counts once the fields outgrow the caches: at 512^3 16 x 16 blocks move 24 GB of HBM
+// traffic per launch (their neighbours' halo lines have left L2 when they come to them) and take
+// 4.4 ms, 64 x 8 ones 14 GB and 3.58 ms, 32 x 16 ones 3.68; 256^3 0.528 / 0.474 ms, 192 x 160 x 128 127 /
+// 118 us, 128^3 58.1 / 56.9 us. Below that the narrow block's finer grain is worth more (96^3 31.0 / 37.8
+// us, 32 x 16 33.6). Above, the tiles that cover the region at the least cost: 16 x 16 against 32 x 16
+// 352^3 1619 / 1255 us, 224^3 402 / 356, 160^3 137 / 126, 416 x 96 x 96 126 / 118.
+//
+// FP64 (256 columns a block) chooses between 16 x 16 and 32 x 8, which takes 2 to 3 % longer on what both
+// cover alike (128^3 121 / 118 us, 512^3 7.41 / 7.30 ms), by the cost of their z-chunks: 150 x 33 x 110 (30
+// or 25 tiles) 47.2 / 42.5 us, 160 x 40 x 200 76.9 / 69.3; 64 x 24 x 64 (8 or 6, all resident either way)
+// 16.0 / 17.4.
+static int2
+ring_tile(int nx, int ny, int nz)
+{
+    const int2 narrow = make_int2(16, 16);
+#if AC_DOUBLE_PRECISION == 1
+    const int2 flat = make_int2(32, 8);
+    return 1.03 * ring_plan(flat, nx, ny, nz).cost < ring_plan(narrow, nx, ny, nz).cost ? flat : narrow;
+#else
+    if ((long)nx * ny * nz < 1L << 21)
+        return narrow;
+    auto up = [](long n, long t) { return (n + t - 1) / t * t; };
+    auto of = [&](int2 t, long cost) { return up(nx, t.x) * up(ny, t.y) * cost; }; // cost per cell of the tiles
+    const int2 flat = make_int2(64, 8), tall = make_int2(32, 16);
+    const int2 wide = of(tall, 103) < of(flat, 100) ? tall : flat;
+    return of(wide, wide.x == 32 ? 103 : 100) < of(narrow, 112) ? wide : narrow;
+#endif
+}
+
+// z-depth of the ring march over nx x ny x nz cells (0: whole columns).
+static int
+ring_z_depth(int nx, int ny, int nz)
+{
+    const int zd = ring_plan(ring_tile(nx, ny, nz), nx, ny, nz).zdepth;
+    return zd >= nz ? 0 : zd;
 }
 
 AcKernelConfig
@@ -1861,12 +1879,15 @@ template <bool COMP>
 static hipError_t
 launch_ring_tile(const SubstepArgs& a, int zdepth, hipStream_t stream)
 {
-#if AC_DOUBLE_PRECISION == 0
     const int2 tile = ring_tile(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z);
+#if AC_DOUBLE_PRECISION == 0
     if (tile.x == 64)
         return launch_ring<64, 8, COMP>(a, zdepth, stream);
     if (tile.x == 32)
         return launch_ring<32, 16, COMP>(a, zdepth, stream);
+#else
+    if (tile.x == 32)
+        return launch_ring<32, 8, COMP>(a, zdepth, stream);
 #endif
     return launch_ring<16, 16, COMP>(a, zdepth, stream);
 }

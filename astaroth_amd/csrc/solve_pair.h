@@ -33,10 +33,10 @@ template <int TX, int TY, bool COMP> struct ZMarchPair {
     static constexpr int NG = NF / 2; // fields of a group: a vector and a scalar, in this order
     static constexpr int LX = TX + 6, LY = TY + 6, LN = LX * LY;
     static constexpr int R     = (LN + NC - 1) / NC; // staging rounds per field and plane
-    // One tile row, in field pairs: a multiple of 256 bytes, so that 16 lanes of one row and 16 of the
-    // next, which a 16-byte read serves together, lie in different banks (88 pairs, unpadded: 64^3 in
-    // whole columns 199 us, 96: 180).
-    static constexpr int PITCH = (NF / 2 * LX + 15) / 16 * 16;
+    // One tile row, in field pairs. With 16-wide tiles a multiple of 256 bytes, so that 16 lanes of one row
+    // and 16 of the next, which a 16-byte read serves together, lie in different banks (88 pairs,
+    // unpadded: 64^3 in whole columns 199 us, 96: 180). A wider tile's row fills the banks by itself.
+    static constexpr int PITCH = TX % 32 ? (NF / 2 * LX + 15) / 16 * 16 : NF / 2 * LX;
 
     // Two fields of a cell. A group's pairs: vector x and y; vector z and the scalar.
     typedef AcReal Two __attribute__((ext_vector_type(2)));

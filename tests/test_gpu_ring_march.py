@@ -139,3 +139,30 @@ def test_ring_march_tiles(dims):
         for q in range(8):
             assert np.abs(out[0][q]).max() > 0
             assert np.array_equal(out[1][q], out[0][q]) and np.array_equal(out[2][q], out[0][q]), (dims, compensated, q)
+
+
+@pytest.mark.parametrize("compensated", [False, True], ids=["plain", "compensated"])
+@pytest.mark.parametrize("dims", [(150, 33, 60), (145, 35, 61)], ids=lambda d: "%dx%dx%d" % d)
+def test_ring_march_fp64_flat_tiles(dims, compensated):
+    """FP64 regions that 32 x 8 tiles cover at less cost than 16 x 16 ones, against the oracle
+    (tolerance as above)."""
+    nx, ny, nz = dims
+    lib = Library(True)
+    info = lib.config(n=nx, ny=ny, nz=nz)
+    fields = mhd_fields(nx, ny, nz, np.float64, config_id=6)
+    ref = [f.copy() for f in fields]
+    pyoracle.integrate_steps_gpu_form(ref, real_params_double(info), DT, 2)
+    for depth in (0, 2):
+        with lib.device_create(0, info, autotune=False) as dev:
+            dev.set_kernel_config(8, 16, 16, depth)
+            dev.set_compensated_integration(compensated)
+            mesh = HostMesh(lib, info, [f.copy() for f in fields])
+            dev.load_mesh(mesh)
+            for _ in range(2):
+                dev.integrate_step(DT)
+            out = mesh.copy()
+            dev.store_mesh(out)
+        for q in range(8):
+            want = ref[q][3:-3, 3:-3, 3:-3]
+            scale = max(np.abs(want).max(), np.abs(fields[q]).max())
+            assert np.abs(out.interior(q) - want).max() <= 24 * np.finfo(np.float64).eps * scale, (dims, depth, q)
