@@ -107,7 +107,8 @@ bool batch_tile_supported(int tile_x, int tile_y);
 // Blocks of the batched solve build for this tile that are resident at once on the current
 // device (occupancy per CU x CUs), or -1 on error.
 int batch_resident_blocks(int tile_x, int tile_y);
-hipError_t launch_substep_batch(int tile_x, int tile_y, const SubstepArgs* boxes,
+// `step`: the substep that every box's arguments are for.
+hipError_t launch_substep_batch(int tile_x, int tile_y, int step, const SubstepArgs* boxes,
                                 const BatchItem* items, int nitems, int nblocks,
                                 hipStream_t stream);
 int kernel_config_count();

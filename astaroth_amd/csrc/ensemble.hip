@@ -537,7 +537,7 @@ enqueue_step(Ensemble e, int par0)
     // fill; one fill after the last substep leaves every box's ghosts current.
     int par = par0;
     for (int s = 0; s < 3; ++s) {
-        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, e->d_args[s][par], e->d_items,
+        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, s, e->d_args[s][par], e->d_items,
                                           e->nitems, e->nblocks, e->stream));
         par = 1 - par;
     }
@@ -552,23 +552,23 @@ valid_dt(AcReal dt)
     return std::isfinite((double)dt) && dt > 0;
 }
 
-// Shortest of `samples` launches of substep 0 of the batched solve over the current work list,
-// after `warm` untimed ones. Substep 0 reads the current set and writes the other one, which
-// holds no state between steps.
+// Shortest of `samples` launches of substep 1 of the batched solve over the current work list,
+// after `warm` untimed ones (two of a step's three launches read a previous stage, substep 0 does
+// not). It reads the current set and rewrites the other one, which holds no state between steps.
 float
 time_batch(Ensemble e, int warm, int samples)
 {
     hipEvent_t t0, t1;
     AC_HIP_CHECK(hipEventCreate(&t0));
     AC_HIP_CHECK(hipEventCreate(&t1));
-    const SubstepArgs* args = e->d_args[0][e->parity];
+    const SubstepArgs* args = e->d_args[1][e->parity];
     for (int i = 0; i < warm; ++i)
-        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, args, e->d_items, e->nitems,
+        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, 1, args, e->d_items, e->nitems,
                                           e->nblocks, e->stream));
     float best = INFINITY;
     for (int i = 0; i < samples; ++i) {
         AC_HIP_CHECK(hipEventRecord(t0, e->stream));
-        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, args, e->d_items, e->nitems,
+        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, 1, args, e->d_items, e->nitems,
                                           e->nblocks, e->stream));
         AC_HIP_CHECK(hipEventRecord(t1, e->stream));
         AC_HIP_CHECK(hipEventSynchronize(t1));

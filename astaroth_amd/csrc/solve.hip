@@ -1638,14 +1638,14 @@ launch_direct(const SubstepArgs& a, hipStream_t stream)
 
 
 // Two waves per SIMD in both precisions (FP64 blocks have two threads per cell column).
-template <int TX, int TY, bool COMP>
-__global__ void __launch_bounds__((RingColumn<TX, TY, COMP>::NT)) __attribute__((amdgpu_waves_per_eu(2)))
+template <int TX, int TY, bool COMP, bool FIRST>
+__global__ void __launch_bounds__((RingColumn<TX, TY, COMP, FIRST>::NT)) __attribute__((amdgpu_waves_per_eu(2)))
 solve_ring(const SubstepArgs a, const int zdepth, const int ntx, const int nty)
 {
-    __shared__ typename RingColumn<TX, TY, COMP>::Shared sh;
+    __shared__ typename RingColumn<TX, TY, COMP, FIRST>::Shared sh;
     int btx, bty, btz;
     strip_tile(xcd_remap((int)blockIdx.x, (int)gridDim.x), ntx, nty, btx, bty, btz);
-    ring_column<TX, TY, COMP>(a, sh, btx, bty, a.start.z + btz * zdepth, zdepth);
+    ring_column<TX, TY, COMP, FIRST>(a, sh, btx, bty, a.start.z + btz * zdepth, zdepth);
 }
 
 template <int TX, int TY, bool COMP>
@@ -1654,7 +1654,8 @@ launch_ring(const SubstepArgs& a, int zdepth, hipStream_t stream)
 {
     if (!fields_equally_spaced(a))
         return hipErrorInvalidValue;
-    return launch_zmarch_grid<TX, TY>(solve_ring<TX, TY, COMP>, a, zdepth, stream, RingColumn<TX, TY, COMP>::NT);
+    const ZMarchKernel kernel = a.rk.step == 0 ? solve_ring<TX, TY, COMP, true> : solve_ring<TX, TY, COMP, false>;
+    return launch_zmarch_grid<TX, TY>(kernel, a, zdepth, stream, RingColumn<TX, TY, COMP, false>::NT);
 }
 
 // Persistent form for ensembles of independent boxes: a grid sized to the resident block slots
@@ -1668,30 +1669,31 @@ launch_ring(const SubstepArgs& a, int zdepth, hipStream_t stream)
 // Slot s takes items s, s + G, s + 2 G, ... (G = gridDim.x) up to its first empty one (box < 0);
 // slots are numbered so that each XCD has a contiguous range (xcd_remap): neighbouring slots mostly
 // hold neighbouring tile columns of one box, whose halo lines are then shared in one L2.
-template <int TX, int TY>
-__global__ void __launch_bounds__((RingColumn<TX, TY, false>::NT)) __attribute__((amdgpu_waves_per_eu(2)))
+template <int TX, int TY, bool FIRST>
+__global__ void __launch_bounds__((RingColumn<TX, TY, false, FIRST>::NT)) __attribute__((amdgpu_waves_per_eu(2)))
 solve_ring_batch(const SubstepArgs* __restrict__ boxes, const BatchItem* __restrict__ items,
                  const int nitems)
 {
-    __shared__ typename RingColumn<TX, TY, false>::Shared sh;
+    __shared__ typename RingColumn<TX, TY, false, FIRST>::Shared sh;
     for (int it = xcd_remap((int)blockIdx.x, (int)gridDim.x); it < nitems; it += gridDim.x) {
         const BatchItem w = items[it];
         if (w.box < 0)
             break;
         const SubstepArgs a = boxes[w.box];
-        ring_column<TX, TY, false>(a, sh, w.btx, w.bty, w.zs, w.zdepth);
+        ring_column<TX, TY, false, FIRST>(a, sh, w.btx, w.bty, w.zs, w.zdepth);
     }
 }
 
 #if AC_DOUBLE_PRECISION == 0
 // The same with 512-thread blocks, each box in 64 x 8 or 32 x 16 tiles (BatchItem::tall).
+template <bool FIRST>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 solve_ring_batch_wide(const SubstepArgs* __restrict__ boxes, const BatchItem* __restrict__ items,
                       const int nitems)
 {
     __shared__ union {
-        RingColumn<64, 8, false>::Shared flat;
-        RingColumn<32, 16, false>::Shared tall;
+        RingColumn<64, 8, false, FIRST>::Shared flat;
+        RingColumn<32, 16, false, FIRST>::Shared tall;
     } sh;
     for (int it = xcd_remap((int)blockIdx.x, (int)gridDim.x); it < nitems; it += gridDim.x) {
         const BatchItem w = items[it];
@@ -1699,9 +1701,9 @@ solve_ring_batch_wide(const SubstepArgs* __restrict__ boxes, const BatchItem* __
             break;
         const SubstepArgs a = boxes[w.box];
         if (w.tall)
-            ring_column<32, 16, false>(a, sh.tall, w.btx, w.bty, w.zs, w.zdepth);
+            ring_column<32, 16, false, FIRST>(a, sh.tall, w.btx, w.bty, w.zs, w.zdepth);
         else
-            ring_column<64, 8, false>(a, sh.flat, w.btx, w.bty, w.zs, w.zdepth);
+            ring_column<64, 8, false, FIRST>(a, sh.flat, w.btx, w.bty, w.zs, w.zdepth);
     }
 }
 #endif
@@ -2018,33 +2020,34 @@ batch_tile_supported(int tx, int ty)
 
 typedef void (*BatchKernel)(const SubstepArgs*, const BatchItem*, int);
 
+template <bool FIRST>
 static BatchKernel
 batch_kernel(int tx, int ty)
 {
 #if AC_DOUBLE_PRECISION == 0
     if (tx == 64 && ty == 8)
-        return solve_ring_batch_wide;
+        return solve_ring_batch_wide<FIRST>;
 #endif
     if (tx == 32 && ty == 4)
-        return solve_ring_batch<32, 4>;
+        return solve_ring_batch<32, 4, FIRST>;
     if (tx == 16 && ty == 8)
-        return solve_ring_batch<16, 8>;
+        return solve_ring_batch<16, 8, FIRST>;
     if (tx == 16 && ty == 16)
-        return solve_ring_batch<16, 16>;
+        return solve_ring_batch<16, 16, FIRST>;
     return nullptr;
 }
 
 static int
 batch_threads(int tx, int ty)
 {
-    return tx * ty * (RingColumn<16, 16, false>::NT / 256);
+    return tx * ty * (RingColumn<16, 16, false, false>::NT / 256);
 }
 
 hipError_t
-launch_substep_batch(int tx, int ty, const SubstepArgs* boxes, const BatchItem* items, int nitems,
+launch_substep_batch(int tx, int ty, int step, const SubstepArgs* boxes, const BatchItem* items, int nitems,
                      int nblocks, hipStream_t stream)
 {
-    const BatchKernel kernel = batch_kernel(tx, ty);
+    const BatchKernel kernel = step == 0 ? batch_kernel<true>(tx, ty) : batch_kernel<false>(tx, ty);
     if (!kernel || nblocks <= 0 || nitems <= 0)
         return hipErrorInvalidConfiguration;
     kernel<<<dim3(nblocks), dim3(batch_threads(tx, ty)), 0, stream>>>(boxes, items, nitems);
@@ -2054,7 +2057,7 @@ launch_substep_batch(int tx, int ty, const SubstepArgs* boxes, const BatchItem* 
 int
 batch_resident_blocks(int tx, int ty)
 {
-    const BatchKernel kernel = batch_kernel(tx, ty);
+    const BatchKernel kernel = batch_kernel<false>(tx, ty);
     int per_cu = 0, cus = 0, dev = 0;
     if (!kernel || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, batch_threads(tx, ty), 0) != hipSuccess ||
         hipGetDevice(&dev) != hipSuccess ||

@@ -27,7 +27,8 @@ namespace {
 // As in the other march, every multiply-add is written out.
 #pragma clang fp contract(off)
 
-template <int TX, int TY, bool COMP> struct ZMarchPair {
+// FIRST: the build of substep 0, which has no previous stage.
+template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
     static constexpr int NC = TX * TY, NT = 2 * NC; // cell columns, threads
     static_assert(NC % 64 == 0, "whole waves");
     static constexpr int NG = NF / 2; // fields of a group: a vector and a scalar, in this order
@@ -56,8 +57,9 @@ template <int TX, int TY, bool COMP> struct ZMarchPair {
         // its second derivatives along each component's own axis and along the other two, and the cross
         // derivatives of grad div, which the second derivatives join last: they are the largest terms
         AcReal own[3], rest[3], gd[3];
-        AcReal prev[NG];    // output z: previous stage
-        AcReal cin[COMP ? NG : 1], cprev[COMP ? NG : 1]; // and its rounding errors (compensated integration)
+        AcReal prev[FIRST ? 1 : NG];           // output z: previous stage
+        AcReal cin[COMP ? NG : 1];             // rounding errors (compensated integration),
+        AcReal cprev[COMP && !FIRST ? NG : 1]; // and those of the previous stage
         int s0, s1, s2, s3; // first element of the ring slots of planes z..z+3 (uniform)
     };
 
@@ -75,7 +77,6 @@ template <int TX, int TY, bool COMP> struct ZMarchPair {
     int group;   // 0: flow, 1: field (uniform in a wave)
     int image;   // ghost planes: n_z where they are read at their periodic images, else 0
     long fs, fv; // field 0 to the group's scalar and to its vector, in cells
-    const AcReal *before, *cbefore; // field 0 of the previous stage and of its rounding errors
     unsigned own;
     bool active;
     unsigned goff[R]; // byte offset in a plane of what this thread stages, per round
@@ -401,17 +402,19 @@ template <int TX, int TY, bool COMP> struct ZMarchPair {
         return l;
     }
 
-    // The previous stage at output plane z, a whole step before it is used (substep 0: the current
-    // values, whose difference to themselves vanishes).
+    // The previous stage at output plane z, a whole step before it is used.
     __device__ __forceinline__ void load_prev(State& st, int z) const
     {
+        if (FIRST && !COMP)
+            return;
         const unsigned long oz = (unsigned long)min(z, ze - 1) * a.mxy;
         const unsigned ow      = pin(own);
-        each(before + oz, [&](int n, const AcReal* p) { st.prev[n] = ld(p, ow); });
-        if (COMP) {
+        if (!FIRST)
+            each(a.out[0] + oz, [&](int n, const AcReal* p) { st.prev[n] = ld(p, ow); });
+        if (COMP)
             each(a.cin[0] + oz, [&](int n, const AcReal* p) { st.cin[n] = ld(p, ow); });
-            each(cbefore + oz, [&](int n, const AcReal* p) { st.cprev[n] = ld(p, ow); });
-        }
+        if (COMP && !FIRST)
+            each(a.cout[0] + oz, [&](int n, const AcReal* p) { st.cprev[n] = ld(p, ow); });
     }
 
     // The groups' rates (mhd_rates_lean in two parts): rate[0..2] of the vector, rate[3] of the scalar.
@@ -540,15 +543,16 @@ template <int TX, int TY, bool COMP> struct ZMarchPair {
             const AcReal u = st.cur[f];
             if (COMP) { // the pair (u, c), as in ZMarchRing
                 const AcReal ci   = st.cin[f];
-                const AcReal diff = (u - st.prev[f]) + (ci - st.cprev[f]);
-                const AcReal d    = mad(K.beta, mad(K.dt, rate[f], K.ab * diff), ci);
+                const AcReal incr = FIRST ? K.dt * rate[f]
+                                          : mad(K.dt, rate[f], K.ab * ((u - st.prev[f]) + (ci - st.cprev[f])));
+                const AcReal d    = mad(K.beta, incr, ci);
                 const AcReal sum  = u + d;
                 const AcReal bb   = sum - u;
                 err[f]            = (u - (sum - bb)) + (d - bb);
                 res[f]            = sum;
             }
             else // the smaller product is the one that is rounded by itself
-                res[f] = mad(K.beta, mad(K.dt, rate[f], K.ab * (u - st.prev[f])), u);
+                res[f] = mad(K.beta, FIRST ? K.dt * rate[f] : mad(K.dt, rate[f], K.ab * (u - st.prev[f])), u);
             settle(res[f]);
         }
         load_prev(st, z + 1);
@@ -619,15 +623,15 @@ template <int TX, int TY, bool COMP> struct ZMarchPair {
     }
 };
 
-template <int TX, int TY, bool COMP> using RingColumn = ZMarchPair<TX, TY, COMP>;
+template <int TX, int TY, bool COMP, bool FIRST> using RingColumn = ZMarchPair<TX, TY, COMP, FIRST>;
 
 // One z-march column: tile (btx, bty) of box `a`, output planes [zs, min(zs + zdepth, end.z)).
-template <int TX, int TY, bool COMP>
+template <int TX, int TY, bool COMP, bool FIRST>
 __device__ __forceinline__ void
-ring_column(const SubstepArgs& a, typename ZMarchPair<TX, TY, COMP>::Shared& sh, const int btx, const int bty,
+ring_column(const SubstepArgs& a, typename ZMarchPair<TX, TY, COMP, FIRST>::Shared& sh, const int btx, const int bty,
             const int zs, const int zdepth)
 {
-    typedef ZMarchPair<TX, TY, COMP> K;
+    typedef ZMarchPair<TX, TY, COMP, FIRST> K;
     K k(a, sh);
     k.group       = __builtin_amdgcn_readfirstlane((int)threadIdx.x / K::NC);
     const int tid = (int)threadIdx.x - k.group * K::NC;
@@ -638,8 +642,6 @@ ring_column(const SubstepArgs& a, typename ZMarchPair<TX, TY, COMP>::Shared& sh,
     const int x0 = a.start.x + btx * TX, y0 = a.start.y + bty * TY;
     const int gx = x0 + tx, gy = y0 + ty;
     k.ze     = min(zs + zdepth, a.end.z);
-    k.before  = a.rk.step == 0 ? a.in[0] : a.out[0];
-    k.cbefore = a.rk.step == 0 ? a.cin[0] : a.cout[0];
     k.image  = a.wrap ? a.mz - 2 * NGHOST : 0;
     k.active = gx < a.end.x && gy < a.end.y;
     k.own    = (unsigned)(k.active ? gx + gy * a.mx : x0 + y0 * a.mx) * sizeof(AcReal);

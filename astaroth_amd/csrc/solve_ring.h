@@ -42,7 +42,8 @@ namespace {
 // block's column begins.
 #pragma clang fp contract(off)
 
-template <int TX, int TY, bool COMP> struct ZMarchRing {
+// FIRST: the build of substep 0, which has no previous stage.
+template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchRing {
     static constexpr int NT = TX * TY;
     static_assert(NT % 64 == 0, "whole waves");
     static constexpr int LX = TX + 6, LY = TY + 6, LN = LX * LY;
@@ -63,8 +64,9 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
         // grad div A - lap A (the other two axes) last: they are the largest terms, and what is
         // added to them is rounded at their size.
         AcReal own[3], rest[3];
-        AcReal prev[NF];  // output z: previous stage
-        AcReal cin[COMP ? NF : 1], cprev[COMP ? NF : 1]; // and its rounding errors (compensated integration)
+        AcReal prev[FIRST ? 1 : NF];                   // output z: previous stage
+        AcReal cin[COMP ? NF : 1];                     // rounding errors (compensated integration),
+        AcReal cprev[COMP && !FIRST ? NF : 1];         // and those of the previous stage
         int s0, s1, s2, s3; // first element of the ring slots of planes z..z+3 (uniform)
     };
 
@@ -72,7 +74,6 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
     Shared& sh;
     int cofs, ze;
     int image; // ghost planes: n_z where they are read at their periodic images, else 0
-    const AcReal *before, *cbefore; // field 0 of the previous stage and of its rounding errors
     unsigned own;
     bool active;
     unsigned goff[R]; // byte offset in a plane of what this thread stages, per round
@@ -453,27 +454,32 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
         return line(c, m);
     }
 
-    // The previous stage at output plane z, a whole step before it is used. Substep 0 has none and
-    // reads the current values instead, whose difference to themselves vanishes: the same code
-    // without a branch.
+    // The previous stage at output plane z, a whole step before it is used.
     __device__ __forceinline__ void load_prev(State& st, int z) const
     {
+        if (FIRST && !COMP)
+            return;
         const unsigned long oz = (unsigned long)min(z, ze - 1) * a.mxy;
-        const AcReal* src      = before + oz;
         const long stride      = field_stride();
         const unsigned ow      = pin(own);
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            st.prev[f] = ld(src, ow);
-            src += stride;
-        }
-        if (COMP) {
-            const AcReal *ci = a.cin[0] + oz, *cp = cbefore + oz;
+        if (!FIRST) {
+            const AcReal* src = a.out[0] + oz;
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
-                st.cin[f]   = ld(ci, ow);
-                st.cprev[f] = ld(cp, ow);
-                ci += stride, cp += stride;
+                st.prev[f] = ld(src, ow);
+                src += stride;
+            }
+        }
+        if (COMP) {
+            const AcReal *ci = a.cin[0] + oz, *cp = a.cout[0] + oz;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                st.cin[f] = ld(ci, ow);
+                ci += stride;
+                if (!FIRST) {
+                    st.cprev[f] = ld(cp, ow);
+                    cp += stride;
+                }
             }
         }
     }
@@ -567,17 +573,19 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
                 //   d = beta (ab ((u_in - u_prev) + (c_in - c_prev)) + dt F) + c_in,
                 // and added with an error-free two-sum (Knuth's TwoSum), whose error term is the
                 // new compensation: u_out + c_out = u_in + d exactly. The stencils read u only.
-                const AcReal ci = st.cin[f];
-                const AcReal diff = (u - st.prev[f]) + (ci - st.cprev[f]);
-                const AcReal d    = mad(a.rk.beta, mad(a.rk.dt, rate[f], a.rk.ab * diff), ci);
-                const AcReal sum = u + d;
-                const AcReal bb  = sum - u;
-                err[f]           = (u - (sum - bb)) + (d - bb);
-                res[f]           = sum;
+                const AcReal ci   = st.cin[f];
+                const AcReal incr = FIRST ? a.rk.dt * rate[f]
+                                          : mad(a.rk.dt, rate[f], a.rk.ab * ((u - st.prev[f]) + (ci - st.cprev[f])));
+                const AcReal d    = mad(a.rk.beta, incr, ci);
+                const AcReal sum  = u + d;
+                const AcReal bb   = sum - u;
+                err[f]            = (u - (sum - bb)) + (d - bb);
+                res[f]            = sum;
             }
             else
                 // the smaller product is the one that is rounded by itself
-                res[f] = mad(a.rk.beta, mad(a.rk.dt, rate[f], a.rk.ab * (u - st.prev[f])), u);
+                res[f] = mad(a.rk.beta,
+                             FIRST ? a.rk.dt * rate[f] : mad(a.rk.dt, rate[f], a.rk.ab * (u - st.prev[f])), u);
             settle(res[f]);
         }
         load_prev(st, z + 1);
@@ -652,23 +660,21 @@ template <int TX, int TY, bool COMP> struct ZMarchRing {
     }
 };
 
-template <int TX, int TY, bool COMP> using RingColumn = ZMarchRing<TX, TY, COMP>;
+template <int TX, int TY, bool COMP, bool FIRST> using RingColumn = ZMarchRing<TX, TY, COMP, FIRST>;
 
 // One z-march column: tile (btx, bty) of box `a`, output planes [zs, min(zs + zdepth, end.z)).
-template <int TX, int TY, bool COMP>
+template <int TX, int TY, bool COMP, bool FIRST>
 __device__ __forceinline__ void
-ring_column(const SubstepArgs& a, typename ZMarchRing<TX, TY, COMP>::Shared& sh, const int btx, const int bty,
+ring_column(const SubstepArgs& a, typename ZMarchRing<TX, TY, COMP, FIRST>::Shared& sh, const int btx, const int bty,
             const int zs, const int zdepth)
 {
-    typedef ZMarchRing<TX, TY, COMP> K;
+    typedef ZMarchRing<TX, TY, COMP, FIRST> K;
     K k(a, sh);
     const int tid = threadIdx.x;
     const int tx = tid % TX, ty = tid / TX;
     const int x0 = a.start.x + btx * TX, y0 = a.start.y + bty * TY;
     const int gx = x0 + tx, gy = y0 + ty;
     k.ze     = min(zs + zdepth, a.end.z);
-    k.before  = a.rk.step == 0 ? a.in[0] : a.out[0];
-    k.cbefore = a.rk.step == 0 ? a.cin[0] : a.cout[0];
     k.image  = a.wrap ? a.mz - 2 * NGHOST : 0;
     k.active = gx < a.end.x && gy < a.end.y;
     k.own    = (unsigned)(k.active ? gx + gy * a.mx : x0 + y0 * a.mx) * sizeof(AcReal);
