@@ -417,18 +417,18 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
             each(a.cout[0] + oz, [&](int n, const AcReal* p) { st.cprev[n] = ld(p, ow); });
     }
 
-    // The groups' rates (mhd_rates_lean in two parts): rate[0..2] of the vector, rate[3] of the scalar.
-    // `os` is the other group's scalar, `ov` its vector; each sends what the other needs half way.
-    __device__ __forceinline__ void flow_rates(const State& st, AcReal os, const Constants& K, AcReal* rate) const
+    // The groups' rates (mhd_rates_lean in two parts), before and after the barrier that both groups share
+    // (in finish): what the other group needs is sent first; `keep` is what a group goes on with.
+    // `os` is the other group's scalar, `u` its vector; rate[0..2] of the vector, rate[3] of the scalar.
+    __device__ __forceinline__ void flow_send(const State& st, AcReal os, const Constants& K, AcReal (&keep)[9]) const
     {
         const AcReal(&ug)[3][3] = st.vg;
-        const AcReal *lg = st.sg, *u = st.cur, lr = st.cur[3];
+        const AcReal *lg = st.sg, lr = st.cur[3];
         const AcReal divu = ug[0][0] + ug[1][1] + ug[2][2];
         const AcReal t    = AcReal(2. / 3.) * divu;
         const AcReal D00 = mad(AcReal(2), ug[0][0], -t), D11 = mad(AcReal(2), ug[1][1], -t),
                      D22 = mad(AcReal(2), ug[2][2], -t);
         const AcReal D01 = ug[0][1] + ug[1][0], D02 = ug[0][2] + ug[2][0], D12 = ug[1][2] + ug[2][1];
-        const AcReal D[3][3] = {{D00, D01, D02}, {D01, D11, D12}, {D02, D12, D22}};
         const AcReal rho     = fast_exp<AcReal>(lr);
         const AcReal inv_rho = fast_rcp<AcReal>(rho);
         const AcReal E       = fast_exp<AcReal>(mad(K.gamma_inv_cp, os, K.gamma_m1 * (lr - K.lnrho0)));
@@ -440,7 +440,16 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
         AcReal* x            = &sh.flow[0][lane];
         x[0] = rho * shear, x[NC] = inv_rho, x[2 * NC] = inv_pT;
         x[3 * NC] = lg[0], x[4 * NC] = lg[1], x[5 * NC] = lg[2], x[6 * NC] = st.slap;
-        __syncthreads();
+        keep[0] = D00, keep[1] = D11, keep[2] = D22, keep[3] = D01, keep[4] = D02, keep[5] = D12;
+        keep[6] = divu, keep[7] = inv_rho, keep[8] = cs2;
+    }
+    __device__ __forceinline__ void flow_rates(const State& st, const Constants& K, const AcReal (&keep)[9],
+                                               AcReal* rate) const
+    {
+        const AcReal(&ug)[3][3] = st.vg;
+        const AcReal *lg = st.sg, *u = st.cur;
+        const AcReal D[3][3] = {{keep[0], keep[3], keep[4]}, {keep[3], keep[1], keep[5]}, {keep[4], keep[5], keep[2]}};
+        const AcReal divu = keep[6], inv_rho = keep[7], cs2 = keep[8];
         const AcReal* y     = &sh.field[0][lane];
         const AcReal jxB[3] = {y[0], y[NC], y[2 * NC]}, sg[3] = {y[3 * NC], y[4 * NC], y[5 * NC]};
         rate[3]             = -mad(u[2], lg[2], mad(u[1], lg[1], u[0] * lg[0])) - divu;
@@ -458,7 +467,7 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
             rate[r]   = mad(K.zeta, gdu, du);
         }
     }
-    __device__ __forceinline__ void field_rates(const State& st, const AcReal* u, const Constants& K, AcReal* rate) const
+    __device__ __forceinline__ void field_send(const State& st, const Constants& K, AcReal (&keep)[9]) const
     {
         const AcReal(&ag)[3][3] = st.vg;
         const AcReal* sg        = st.sg;
@@ -472,7 +481,14 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
         x[NC]     = mad(j[2], B[0], -(j[0] * B[2]));
         x[2 * NC] = mad(j[0], B[1], -(j[1] * B[0]));
         x[3 * NC] = sg[0], x[4 * NC] = sg[1], x[5 * NC] = sg[2];
-        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+            keep[r] = B[r], keep[3 + r] = j[r];
+    }
+    __device__ __forceinline__ void field_rates(const State& st, const AcReal* u, const Constants& K,
+                                                const AcReal (&keep)[9], AcReal* rate) const
+    {
+        const AcReal *sg = st.sg, *B = &keep[0], *j = &keep[3];
         const AcReal* y   = &sh.flow[0][lane];
         const AcReal heat = y[0], inv_rho = y[NC], inv_pT = y[2 * NC], lr_lap = y[6 * NC];
         const AcReal lg[3] = {y[3 * NC], y[4 * NC], y[5 * NC]};
@@ -526,13 +542,17 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
         add_ahead(st.gd, h3, P.cxz[3], P.cyz[3]);
         settle(st.sg[2], st.slap, st.vg[0][2], st.rest[0], st.vg[1][2], st.rest[1], st.vg[2][2], st.own[2]);
         fence();
-        AcReal rate[NG];
+        AcReal rate[NG], keep[9];
+        const AcReal ou[3] = {o0[0], o0[1], o1[0]};
         if (group == 0)
-            flow_rates(st, o1[1], K, rate);
-        else {
-            const AcReal u[3] = {o0[0], o0[1], o1[0]};
-            field_rates(st, u, K, rate);
-        }
+            flow_send(st, o1[1], K, keep);
+        else
+            field_send(st, K, keep);
+        __syncthreads(); // one barrier of the whole block, which no branch between its waves contains
+        if (group == 0)
+            flow_rates(st, K, keep, rate);
+        else
+            field_rates(st, ou, K, keep, rate);
         settle(rate[0], rate[1], rate[2], rate[3]);
         fence();
         b = start(st.s1);
