@@ -312,7 +312,15 @@ wide_tiling(int3 n)
     return plane_cost(flat, n) <= plane_cost(tall, n) ? flat : tall;
 }
 
-constexpr Tiling NARROW{16, 16, 0, 50};
+// Tiles of one shape in every box. A plane of a 16 x 8 or 32 x 4 tile, half of the blocks' threads, takes
+// 27 and 26 in FP32 (32 boxes of 64^3 in 16 x 8 tiles 1.02 ms per step, in 32 x 4 ones 1.04) and 62 in
+// FP64, where 16 x 16 takes 100 (1.61 / 1.98 / 1.99 ms).
+Tiling
+narrow_tiling(int tx, int ty)
+{
+    const int weight = tx * ty == 256 ? (AC_DOUBLE_PRECISION ? 100 : 50) : AC_DOUBLE_PRECISION ? 62 : tx == 16 ? 27 : 26;
+    return {tx, ty, 0, weight};
+}
 
 // Tile shape of the launch. In FP32 a 16 x 16 configuration runs 512-thread blocks if their tiles
 // cost less over the whole ensemble (32 boxes of 48^3, which they cover with a third to spare, take
@@ -325,7 +333,7 @@ launch_shape(const Ensemble e)
         for (const AcMeshInfo& i : e->info) {
             const int3 n = dims_of(i);
             wide += plane_cost(wide_tiling(n), n) * n.z;
-            narrow += plane_cost(NARROW, n) * n.z;
+            narrow += plane_cost(narrow_tiling(16, 16), n) * n.z;
         }
         if (wide < narrow)
             return make_int2(64, 8);
@@ -336,7 +344,7 @@ launch_shape(const Ensemble e)
 Tiling
 box_tiling(int2 launch, int3 n)
 {
-    return launch.x == 64 ? wide_tiling(n) : Tiling{launch.x, launch.y, 0, 1};
+    return launch.x == 64 ? wide_tiling(n) : narrow_tiling(launch.x, launch.y);
 }
 
 struct Deal {
@@ -426,33 +434,52 @@ equal_parts(const Ensemble e, int depth)
     return d;
 }
 
-// z-depths by decreasing promise: the work of the busiest block after the dealing, for columns cut
-// at 2 to 128 planes and whole ones. Fewer, longer items save prologues; more, shorter ones fill the
-// chip and leave less of a tail.
+// A configuration of the batched launch, and its expected time (of a plane of all blocks that a CU holds).
+struct Candidate {
+    int tile_x, tile_y;
+    std::map<int, int> class_depth;
+    double time;
+};
+
+void
+apply(Ensemble e, const Candidate& c)
+{
+    e->tile_x      = c.tile_x;
+    e->tile_y      = c.tile_y;
+    e->z_depth     = 0;
+    e->class_depth = c.class_depth;
+}
+
+// The z-depths of a tile shape by decreasing promise: the work of the busiest block after the dealing,
+// for columns cut at 2 to 128 planes and whole ones. Fewer, longer items save prologues; more, shorter
+// ones fill the chip and leave less of a tail. Leaves the ensemble at the first.
 AcResult
-rank_depths(Ensemble e, std::vector<std::map<int, int>>* ranked)
+rank_depths(Ensemble e, int tile_x, int tile_y, std::vector<Candidate>* ranked)
 {
     AC_HIP_CHECK(hipSetDevice(e->id));
+    e->tile_x         = tile_x;
+    e->tile_y         = tile_y;
+    e->z_depth        = 0;
     const int2 launch = launch_shape(e);
     const int slots   = batch_resident_blocks(launch.x, launch.y);
     if (slots < 1)
         return AC_FAILURE;
-    std::vector<std::pair<long, std::map<int, int>>> all;
+    int cus = 0;
+    AC_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->id));
+    const double per_cu = (double)slots / cus;
+    ranked->clear();
     for (const int depth : {1 << 30, 128, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4, 2}) {
         const std::map<int, int> cut = equal_parts(e, depth);
-        if (!all.empty() && cut == all.back().second)
+        if (!ranked->empty() && cut == ranked->back().class_depth)
             continue;
         e->class_depth = cut;
         const Deal d   = deal_items(e, launch, slots);
-        all.push_back({d.makespan, cut});
+        ranked->push_back({tile_x, tile_y, cut, d.makespan * per_cu});
         if (d.items.size() > 32 * (size_t)slots)
             break; // shorter items only cost more
     }
-    std::stable_sort(all.begin(), all.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
-    ranked->clear();
-    for (const auto& c : all)
-        ranked->push_back(c.second);
-    e->class_depth = ranked->front();
+    std::stable_sort(ranked->begin(), ranked->end(), [](const Candidate& a, const Candidate& b) { return a.time < b.time; });
+    apply(e, ranked->front());
     return AC_SUCCESS;
 }
 
@@ -581,11 +608,11 @@ time_batch(Ensemble e, int warm, int samples)
     return best;
 }
 
-// Tuned z-depths per ensemble composition (device, box sizes in order), kept for the process.
-std::map<std::vector<int>, std::map<int, int>>&
+// Tuned choices per ensemble composition (device, box sizes in order), kept for the process.
+std::map<std::vector<int>, Candidate>&
 tuning_cache()
 {
-    static std::map<std::vector<int>, std::map<int, int>> cache;
+    static std::map<std::vector<int>, Candidate> cache;
     return cache;
 }
 
@@ -630,7 +657,7 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     for (auto& i : e->info)
         acHostUpdateBuiltinParams(&i);
     e->parity   = 0;
-    // 16 x 16 tiles (or the wide ones of launch_shape), the z-depths ranked first until the tuner
+    // 16 x 16 tiles (or the wide ones of launch_shape) at the z-depths ranked first, until the tuner
     // (below) measures this composition
     e->tile_x   = 16;
     e->tile_y   = 16;
@@ -707,11 +734,11 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     AC_HIP_CHECK(hipMalloc((void**)&e->d_results, (size_t)nboxes * NDIAG * sizeof(double)));
     AC_HIP_CHECK(hipMemset(e->d_results, 0, (size_t)nboxes * NDIAG * sizeof(double)));
     AC_HIP_CHECK(hipHostMalloc((void**)&e->h_results, (size_t)nboxes * NDIAG * sizeof(double)));
-    std::vector<std::map<int, int>> ranked;
-    if (rank_depths(e, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
+    std::vector<Candidate> ranked;
+    if (rank_depths(e, 16, 16, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
         return AC_FAILURE;
-    // z-depths measured on this composition, as Devices tune at creation; AC_AUTOTUNE=0 keeps the
-    // first.
+    // Tile shape and z-depths measured on this composition, as Devices tune at creation; AC_AUTOTUNE=0
+    // keeps 16 x 16 tiles at the first depths.
     const char* tune = getenv("AC_AUTOTUNE");
     if (!(tune && tune[0] == '0') && acEnsembleAutoOptimize(e) != AC_SUCCESS)
         return AC_FAILURE;
@@ -785,26 +812,35 @@ acEnsembleAutoOptimize(Ensemble e)
         std::lock_guard<std::mutex> lock(tuning_mutex());
         const auto it = tuning_cache().find(key);
         if (it != tuning_cache().end()) {
-            e->tile_x = e->tile_y = 16;
-            e->z_depth     = 0;
-            e->class_depth = it->second;
+            apply(e, it->second);
             return build_items(e);
         }
     }
     // the timed launches need argument arrays; any dt times the same
     if (!e->args_valid && build_args(e, AcReal(1e-3)) != AC_SUCCESS)
         return AC_FAILURE;
-    e->tile_x = e->tile_y = 16;
-    e->z_depth = 0;
-    std::vector<std::map<int, int>> ranked;
-    if (rank_depths(e, &ranked) != AC_SUCCESS)
-        return AC_FAILURE;
-    ranked.resize(std::min<size_t>(ranked.size(), 4));
-    float best = INFINITY;
+    // Of every tile shape the four most promising depths, unless they are expected to take more than
+    // 1.2 times the best: thin boxes fill a tile of one shape and a part of another's (256 boxes of
+    // 32 x 4 x 64 in FP32: 0.70 ms per step in 16 x 16 tiles, 0.42 in 16 x 8, 0.33 in 32 x 4), and
+    // between shapes the expectation is 10 to 20 % off (500 boxes of 20^3, where 32 x 4 is expected to
+    // be 4 % faster than 16 x 8: 0.94 ms against 0.81).
+    std::vector<Candidate> candidates;
+    double least = INFINITY;
+    for (const int2 tile : {make_int2(16, 16), make_int2(16, 8), make_int2(32, 4)}) {
+        std::vector<Candidate> ranked;
+        if (rank_depths(e, tile.x, tile.y, &ranked) != AC_SUCCESS)
+            return AC_FAILURE;
+        least = std::min(least, ranked.front().time);
+        candidates.insert(candidates.end(), ranked.begin(), ranked.begin() + std::min<size_t>(ranked.size(), 4));
+    }
+    candidates.erase(std::remove_if(candidates.begin(), candidates.end(),
+                                    [=](const Candidate& c) { return c.time > 1.2 * least; }),
+                     candidates.end());
+    float best  = INFINITY;
     size_t keep = 0;
     for (int round = 0; round < 2; ++round) // twice: the clocks still rise during the first
-        for (size_t i = 0; i < ranked.size(); ++i) {
-            e->class_depth = ranked[i];
+        for (size_t i = 0; i < candidates.size(); ++i) {
+            apply(e, candidates[i]);
             if (build_items(e) != AC_SUCCESS)
                 return AC_FAILURE;
             const float ms = time_batch(e, 1, 2);
@@ -813,11 +849,11 @@ acEnsembleAutoOptimize(Ensemble e)
                 keep = i;
             }
         }
-    e->class_depth = ranked[keep];
+    apply(e, candidates[keep]);
     if (build_items(e) != AC_SUCCESS)
         return AC_FAILURE;
     std::lock_guard<std::mutex> lock(tuning_mutex());
-    tuning_cache()[key] = e->class_depth;
+    tuning_cache()[key] = candidates[keep];
     return AC_SUCCESS;
 }
 

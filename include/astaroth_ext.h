@@ -197,12 +197,13 @@ int acEnsembleBoxCount(const Ensemble ensemble);
  * 512 threads in 64x8 or 32x16 tiles where these cover the boxes with little to spare. */
 AcResult acEnsembleSetKernelConfig(Ensemble ensemble, const AcKernelConfig config);
 AcResult acEnsembleGetKernelConfig(const Ensemble ensemble, AcKernelConfig* config);
-/* The ensemble's tuner, run by acEnsembleCreate unless the environment sets AC_AUTOTUNE=0. The
- * z-depths (columns of every size class in equal parts) are ranked by the work of the busiest block
- * after the work items are dealt to the resident blocks; the tuner times the batched launch with the
- * first four and keeps the fastest (without it: the first). Results are kept per composition (device
- * and box sizes) for the process. acEnsembleBoxZDepth gives a box's output planes per work item (0:
- * whole columns). */
+/* The ensemble's tuner, run by acEnsembleCreate unless the environment sets AC_AUTOTUNE=0 (then
+ * 16 x 16 tiles). For each tile shape the z-depths (columns of every size class in equal parts) are
+ * ranked by the work of the busiest block after the work items are dealt to the resident blocks; the
+ * tuner times the batched launch with the first four of each shape that comes within 20 % of the most
+ * promising one and keeps the fastest (without it: the first depths). Results are kept per
+ * composition (device and box sizes) for the process. acEnsembleBoxZDepth gives a box's output planes
+ * per work item (0: whole columns). */
 AcResult acEnsembleAutoOptimize(Ensemble ensemble);
 int acEnsembleBoxZDepth(const Ensemble ensemble, const int box);
 AcResult acEnsembleRandomizeUniform(Ensemble ensemble, const int box,
