@@ -301,10 +301,11 @@ plane_cost(const Tiling& t, int3 n)
 }
 
 // 512-thread blocks (FP32) take 64 x 8 tiles, or 32 x 16 ones in a box where those cover enough
-// fewer cells beyond it. A plane of either, and two of 16 x 16 (as many cells), take 81, 92 and 100:
-// 32 boxes of 64^3 0.836 / 0.933 / 1.002 ms per step (0.11 of it fill and diagnostics), 8 of 128^3
-// 1.69 / 1.78 / 1.97 ms, 16 of 96^3 (64 x 8 tiles cover 128 of 96) 1.93 / 1.65 / 1.87 ms. The wide
-// tiles read fewer halo cells and fewer parts of cache lines, which is what bounds a full chip here.
+// fewer cells beyond it. A plane of either, and two of 16 x 16 (as many cells), take 81, 92 and 98:
+// 32 boxes of 64^3 0.82 ms per step in 64 x 8 tiles and 0.92 in 16 x 16 (0.11 of it fill and
+// diagnostics), 8 of 128^3 1.64 and 1.72; 16 of 96^3, of which 64 x 8 tiles cover 128, 1.58 in 32 x 16
+// and 1.76 in 16 x 16. The wide tiles read fewer halo cells and fewer parts of cache lines, which is
+// what bounds a full chip here.
 Tiling
 wide_tiling(int3 n)
 {
@@ -318,13 +319,13 @@ wide_tiling(int3 n)
 Tiling
 narrow_tiling(int tx, int ty)
 {
-    const int weight = tx * ty == 256 ? (AC_DOUBLE_PRECISION ? 100 : 50) : AC_DOUBLE_PRECISION ? 62 : tx == 16 ? 27 : 26;
+    const int weight = tx * ty == 256 ? (AC_DOUBLE_PRECISION ? 100 : 49) : AC_DOUBLE_PRECISION ? 62 : tx == 16 ? 27 : 26;
     return {tx, ty, 0, weight};
 }
 
 // Tile shape of the launch. In FP32 a 16 x 16 configuration runs 512-thread blocks if their tiles
-// cost less over the whole ensemble (32 boxes of 48^3, which they cover with a third to spare, take
-// 0.494 ms per step in 16 x 16 tiles and 0.556 in 64 x 8).
+// cost less over the whole ensemble (100 boxes of 48^3, which they cover with a third to spare, take
+// 1.43 ms per step in 16 x 16 tiles and 1.52 in 64 x 8).
 int2
 launch_shape(const Ensemble e)
 {
@@ -452,9 +453,10 @@ apply(Ensemble e, const Candidate& c)
 
 // The z-depths of a tile shape by decreasing promise: the work of the busiest block after the dealing,
 // for columns cut at 2 to 128 planes and whole ones. Fewer, longer items save prologues; more, shorter
-// ones fill the chip and leave less of a tail. Leaves the ensemble at the first.
+// ones fill the chip and leave less of a tail. Leaves the ensemble at the first. None, without dealing,
+// where even an even deal of whole columns would take more than `limit`.
 AcResult
-rank_depths(Ensemble e, int tile_x, int tile_y, std::vector<Candidate>* ranked)
+rank_depths(Ensemble e, int tile_x, int tile_y, double limit, std::vector<Candidate>* ranked)
 {
     AC_HIP_CHECK(hipSetDevice(e->id));
     e->tile_x         = tile_x;
@@ -468,6 +470,13 @@ rank_depths(Ensemble e, int tile_x, int tile_y, std::vector<Candidate>* ranked)
     AC_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->id));
     const double per_cu = (double)slots / cus;
     ranked->clear();
+    double even = 0;
+    for (const AcMeshInfo& i : e->info) {
+        const int3 n = dims_of(i);
+        even += (double)plane_cost(box_tiling(launch, n), n) * (PROLOGUE + n.z) / cus;
+    }
+    if (even > limit)
+        return AC_SUCCESS;
     for (const int depth : {1 << 30, 128, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4, 2}) {
         const std::map<int, int> cut = equal_parts(e, depth);
         if (!ranked->empty() && cut == ranked->back().class_depth)
@@ -735,7 +744,7 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     AC_HIP_CHECK(hipMemset(e->d_results, 0, (size_t)nboxes * NDIAG * sizeof(double)));
     AC_HIP_CHECK(hipHostMalloc((void**)&e->h_results, (size_t)nboxes * NDIAG * sizeof(double)));
     std::vector<Candidate> ranked;
-    if (rank_depths(e, 16, 16, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
+    if (rank_depths(e, 16, 16, INFINITY, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
         return AC_FAILURE;
     // Tile shape and z-depths measured on this composition, as Devices tune at creation; AC_AUTOTUNE=0
     // keeps 16 x 16 tiles at the first depths.
@@ -820,21 +829,24 @@ acEnsembleAutoOptimize(Ensemble e)
     if (!e->args_valid && build_args(e, AcReal(1e-3)) != AC_SUCCESS)
         return AC_FAILURE;
     // Of every tile shape the four most promising depths, unless they are expected to take more than
-    // 1.2 times the best: thin boxes fill a tile of one shape and a part of another's (256 boxes of
-    // 32 x 4 x 64 in FP32: 0.70 ms per step in 16 x 16 tiles, 0.42 in 16 x 8, 0.33 in 32 x 4), and
-    // between shapes the expectation is 10 to 20 % off (500 boxes of 20^3, where 32 x 4 is expected to
-    // be 4 % faster than 16 x 8: 0.94 ms against 0.81).
+    // 1.1 times the best: thin boxes fill a tile of one shape and a part of another's (256 boxes of
+    // 32 x 4 x 64 in FP32: 0.70 ms per step in 16 x 16 tiles, 0.42 in 16 x 8, 0.33 in 32 x 4). Between
+    // shapes the expectation is 10 to 20 % off (500 boxes of 20^3, where 32 x 4 is expected to be 4 %
+    // faster than 16 x 8: 0.94 ms against 0.81), but a wider margin times shapes that do not win: 12
+    // boxes of 32 to 128 cells an edge took 9 ms longer to create with 1.2.
     std::vector<Candidate> candidates;
     double least = INFINITY;
     for (const int2 tile : {make_int2(16, 16), make_int2(16, 8), make_int2(32, 4)}) {
         std::vector<Candidate> ranked;
-        if (rank_depths(e, tile.x, tile.y, &ranked) != AC_SUCCESS)
+        if (rank_depths(e, tile.x, tile.y, 1.1 * least, &ranked) != AC_SUCCESS)
             return AC_FAILURE;
+        if (ranked.empty())
+            continue;
         least = std::min(least, ranked.front().time);
         candidates.insert(candidates.end(), ranked.begin(), ranked.begin() + std::min<size_t>(ranked.size(), 4));
     }
     candidates.erase(std::remove_if(candidates.begin(), candidates.end(),
-                                    [=](const Candidate& c) { return c.time > 1.2 * least; }),
+                                    [=](const Candidate& c) { return c.time > 1.1 * least; }),
                      candidates.end());
     float best  = INFINITY;
     size_t keep = 0;
@@ -843,8 +855,9 @@ acEnsembleAutoOptimize(Ensemble e)
             apply(e, candidates[i]);
             if (build_items(e) != AC_SUCCESS)
                 return AC_FAILURE;
-            const float ms = time_batch(e, 1, 2);
-            if (round > 0 && ms < best) {
+            const float ms   = time_batch(e, 1, 2);
+            const bool other = candidates[i].tile_x != candidates[keep].tile_x || candidates[i].tile_y != candidates[keep].tile_y;
+            if (round > 0 && ms < (other ? 0.98f : 1.f) * best) { // (the timings scatter by 1 to 2 %)
                 best = ms;
                 keep = i;
             }

@@ -1674,13 +1674,14 @@ __global__ void __launch_bounds__((RingColumn<TX, TY, false, FIRST>::NT)) __attr
 solve_ring_batch(const SubstepArgs* __restrict__ boxes, const BatchItem* __restrict__ items,
                  const int nitems)
 {
-    __shared__ typename RingColumn<TX, TY, false, FIRST>::Shared sh;
+    constexpr bool LATE = TX * TY == 256; // (tiles of 128 cells are for thin boxes, which share few lines)
+    __shared__ typename RingColumn<TX, TY, false, FIRST, LATE>::Shared sh;
     for (int it = xcd_remap((int)blockIdx.x, (int)gridDim.x); it < nitems; it += gridDim.x) {
         const BatchItem w = items[it];
         if (w.box < 0)
             break;
         const SubstepArgs a = boxes[w.box];
-        ring_column<TX, TY, false, FIRST>(a, sh, w.btx, w.bty, w.zs, w.zdepth);
+        ring_column<TX, TY, false, FIRST, LATE>(a, sh, w.btx, w.bty, w.zs, w.zdepth);
     }
 }
 

@@ -646,10 +646,11 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
     }
 };
 
-template <int TX, int TY, bool COMP, bool FIRST> using RingColumn = ZMarchPair<TX, TY, COMP, FIRST>;
+// LATE is an option of the one-thread form.
+template <int TX, int TY, bool COMP, bool FIRST, bool LATE = false> using RingColumn = ZMarchPair<TX, TY, COMP, FIRST>;
 
 // One z-march column: tile (btx, bty) of box `a`, output planes [zs, min(zs + zdepth, end.z)).
-template <int TX, int TY, bool COMP, bool FIRST>
+template <int TX, int TY, bool COMP, bool FIRST, bool LATE = false>
 __device__ __forceinline__ void
 ring_column(const SubstepArgs& a, typename ZMarchPair<TX, TY, COMP, FIRST>::Shared& sh, const int btx, const int bty,
             const int zs, const int zdepth)

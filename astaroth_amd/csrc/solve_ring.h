@@ -21,7 +21,7 @@
 //   march more in spills than it saved).
 // * The ring rows hold all eight fields of a tile row side by side, so one LDS base register per row
 //   serves every field's x window, and rows a tile row apart start 16 banks apart (16-wide tiles).
-// * The previous stage is loaded a whole plane ahead, the next plane too.
+// * The previous stage is loaded a whole plane ahead, the next plane too (but see LATE).
 // * One field pointer and a stride instead of sixteen pointers, which in this march spilled 78 scalar
 //   registers to lanes of vector ones (50 v_readlane a plane). The rates are
 //   formed with fewer operations (mhd_rates_lean). The vector instruction count is level with the
@@ -43,7 +43,15 @@ namespace {
 #pragma clang fp contract(off)
 
 // FIRST: the build of substep 0, which has no previous stage.
-template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchRing {
+//
+// LATE: the next plane is loaded at the end of a plane's work instead of in its middle, two thirds of a
+// plane ahead of its use instead of a whole one. A block then waits for lines that its neighbours have
+// not fetched yet, which keeps the blocks of 16 x 16 tiles at nearly the same z, where they share halo
+// lines in L2: ensembles on a full chip gain (100 boxes of 48^3 1605 -> 1430 us per step, 20 of 80^3
+// 1300 -> 1184, 256 of 32^3 1088 -> 1046), launches with a block or two per CU are level (4 of 48^3 114
+// -> 111, 4 of 80^3 239 -> 241), 512-thread blocks, whose waves march together anyway, lose (32 of 64^3
+// 816 -> 870).
+template <int TX, int TY, bool COMP, bool FIRST, bool LATE> struct ZMarchRing {
     static constexpr int NT = TX * TY;
     static_assert(NT % 64 == 0, "whole waves");
     static constexpr int LX = TX + 6, LY = TY + 6, LN = LX * LY;
@@ -495,7 +503,8 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchRing {
         MhdAgg& g           = st.g;
         stage(st.s3, st.pv); // the slot of plane z-1, which every thread left before the last barrier
         __syncthreads();
-        load(st.pv, z + 4);
+        if (!LATE)
+            load(st.pv, z + 4);
 
         const LdsReal *r1 = row(st.s1, 0), *r2 = row(st.s2, 0), *r3 = row(st.s3, 0);
         const Above n0 = above(r1, r2, r3, VTXBUF_LNRHO, VTXBUF_UUX, VTXBUF_UUY, VTXBUF_UUZ);
@@ -610,6 +619,8 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchRing {
 #pragma unroll
         for (int f = 0; f < NF; ++f)
             st.q[f][PH] = st.cur[f];
+        if (LATE)
+            load(st.pv, z + 4);
         fence();
         const int s = st.s0;
         st.s0 = st.s1, st.s1 = st.s2, st.s2 = st.s3, st.s3 = s;
@@ -663,15 +674,16 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchRing {
     }
 };
 
-template <int TX, int TY, bool COMP, bool FIRST> using RingColumn = ZMarchRing<TX, TY, COMP, FIRST>;
+template <int TX, int TY, bool COMP, bool FIRST, bool LATE = false>
+using RingColumn = ZMarchRing<TX, TY, COMP, FIRST, LATE>;
 
 // One z-march column: tile (btx, bty) of box `a`, output planes [zs, min(zs + zdepth, end.z)).
-template <int TX, int TY, bool COMP, bool FIRST>
+template <int TX, int TY, bool COMP, bool FIRST, bool LATE = false>
 __device__ __forceinline__ void
-ring_column(const SubstepArgs& a, typename ZMarchRing<TX, TY, COMP, FIRST>::Shared& sh, const int btx, const int bty,
-            const int zs, const int zdepth)
+ring_column(const SubstepArgs& a, typename ZMarchRing<TX, TY, COMP, FIRST, LATE>::Shared& sh, const int btx,
+            const int bty, const int zs, const int zdepth)
 {
-    typedef ZMarchRing<TX, TY, COMP, FIRST> K;
+    typedef ZMarchRing<TX, TY, COMP, FIRST, LATE> K;
     K k(a, sh);
     const int tid = threadIdx.x;
     const int tx = tid % TX, ty = tid / TX;
