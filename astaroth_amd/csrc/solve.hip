@@ -1787,83 +1787,102 @@ current_cu_count()
     return n;
 }
 
-// Equal z-chunks for the ring march over nx x ny x nz cells in `tile`: their depth and the cost. A block
-// costs its planes plus a prologue (six planes to stage, three to scatter) worth `pro` of them;
-// blocks run in rounds of the GPU's resident block slots, and a round that leaves every CU one block
-// of two runs its planes in `light` of the time. Measured (FP32, 16 x 16 blocks, us): 3.1 a plane + 5
-// with two blocks per CU, 2.15 a plane + 3 with one; 64 x 8 blocks 2.85 a plane + 6; FP64 2.5 a
-// plane + 8. Equal chunks keep each XCD's contiguous block range equally loaded.
-struct RingPlan {
-    int zdepth;
-    double cost; // planes of one block
+// Tiles of the ring march, each with the time of a plane (of all blocks that a CU holds) relative to
+// 16 x 16 tiles. FP32 chooses between 64 x 8 and 32 x 16 (512 threads, one block per CU) and 16 x 16 (two
+// per CU): all hold 512 cells per CU. The wide blocks read fewer halo cells and parts of cache lines,
+// and their two waves per SIMD cannot drift apart in z, which is what counts once the fields outgrow
+// the caches: at 512^3 16 x 16 blocks move 24 GB of HBM traffic per launch (their neighbours' halo lines
+// have left L2 when they come to them) and take 4.4 ms, 64 x 8 ones 14 GB and 3.62 ms. FP64 (256 columns a
+// block) has 16 x 16 and 32 x 8, which takes 2 to 3 % longer on what both cover alike (128^3 121 / 118 us,
+// 512^3 7.41 / 7.30 ms).
+struct RingTile {
+    int x, y;
+    double plane;
 };
-static RingPlan
-ring_plan(int2 tile, int nx, int ny, int nz)
+#if AC_DOUBLE_PRECISION == 1
+static constexpr RingTile kRingTiles[] = {{16, 16, 1.0}, {32, 8, 1.03}};
+#else
+static constexpr RingTile kRingTiles[] = {{16, 16, 1.0}, {64, 8, 0.92}, {32, 16, 0.95}};
+#endif
+
+// Time of a launch over nx x ny x nz cells in z-chunks of `zd` planes, in planes of 16 x 16 tiles. A block
+// costs its planes plus a prologue (six planes to stage, three to scatter) worth `pro` of them; blocks
+// run in rounds of the GPU's resident block slots, and a round that leaves every CU one block of two
+// runs its planes in `light` of the time. Measured (FP32, 16 x 16 blocks, us): 3.1 a plane + 5 with two
+// blocks per CU, 2.15 a plane + 3 with one; 64 x 8 blocks 2.85 a plane + 6; FP64 2.5 a plane + 8. In FP32
+// 16 x 16 planes take a fifth longer once the two sets of fields (64 bytes a cell) fill the 256 MB of
+// the last-level cache: 48 x 200 x 400 (246 MB) 1.2, 136^3 (161 MB) 1.01, 352^3 1.2 times the expectation
+// from the wide tiles.
+static double
+ring_cost(const RingTile& t, int nx, int ny, int nz, int zd)
 {
-    const int tx      = tile.x, ty = tile.y;
-    const bool wide   = tx * ty == 512;
-    const int per_cu  = wide || AC_DOUBLE_PRECISION ? 1 : 2;
-    const double pro  = AC_DOUBLE_PRECISION ? 3.3 : wide ? 2.1 : 1.6;
+    const bool wide    = t.x * t.y == 512;
+    const int per_cu   = wide || AC_DOUBLE_PRECISION ? 1 : 2;
+    const double pro   = AC_DOUBLE_PRECISION ? 3.3 : wide ? 2.1 : 1.6;
     const double light = per_cu == 2 ? 0.69 : 1.0;
-    const long cus    = current_cu_count();
-    const long cols   = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
-    const long slots  = per_cu * cus;
-    const long kfill  = std::max(1L, (slots + cols - 1) / cols);
-    const int kmax    = (int)std::min(std::max(12L, 4 * kfill), (long)nz);
-    int best_zd       = nz;
-    double best_cost  = INFINITY;
-    for (int k = 1; k <= kmax; ++k) {
-        const int zd      = (nz + k - 1) / k;
-        const long blocks = cols * ((nz + zd - 1) / zd);
-        const long full = blocks / slots, rest = blocks % slots;
-        const double cost =
-            (zd + pro) * ((double)full + (rest == 0 ? 0.0 : rest <= cus ? light : 1.0));
-        if (cost < best_cost) {
-            best_cost = cost;
-            best_zd   = zd;
+    const double far   = per_cu == 2 && (double)nx * ny * nz * 64 > 240e6 ? 1.2 : 1.0;
+    const long cus     = current_cu_count();
+    const long blocks  = (long)((nx + t.x - 1) / t.x) * ((ny + t.y - 1) / t.y) * ((nz + zd - 1) / zd);
+    const long full = blocks / (per_cu * cus), rest = blocks % (per_cu * cus);
+    return t.plane * far * (zd + pro) * ((double)full + (rest == 0 ? 0.0 : rest <= cus ? light : 1.0));
+}
+
+// Whether the launch over nx x ny x nz cells may run in this tile. In FP32 the wide tiles are for 2^21 cells
+// and more; below, the narrow block's finer grain is worth more (96^3 31.0 us, in 64 x 8 tiles 37.8, in
+// 32 x 16 33.6; 128^3 57.4 / 56.8 / 57.6).
+static bool
+ring_tile_fits(const RingTile& t, int nx, int ny, int nz)
+{
+    return AC_DOUBLE_PRECISION || t.x * t.y == 256 || (long)nx * ny * nz >= 1L << 21;
+}
+
+// The tile of least cost at this z-depth (0: whole columns). Which one covers the region with fewer
+// cells beyond it and which one fills its rounds of blocks both count. FP32, 16 x 16 / 64 x 8 / 32 x 16
+// (us): 352^3 1639 / 1412 / 1263, 224^3 398 / 372 / 357, 300 x 96 x 96 80.9 / 78.9 / 80.1, 400 x 80 x 100
+// 84.6 / 104 / 106 (500 blocks on 512 slots, or 260 on 256). FP64, 16 x 16 / 32 x 8: 150 x 33 x 110 (30 or 25
+// tiles) 47.2 / 42.5, 64 x 24 x 64 (8 or 6, all resident either way) 16.0 / 17.4.
+static RingTile
+ring_tile(int nx, int ny, int nz, int zdepth)
+{
+    const int zd  = zdepth <= 0 ? nz : std::min(zdepth, nz);
+    RingTile best = kRingTiles[0];
+    double cost   = INFINITY;
+    for (const RingTile& t : kRingTiles) {
+        if (!ring_tile_fits(t, nx, ny, nz))
+            continue;
+        const double c = ring_cost(t, nx, ny, nz, zd);
+        if (c < cost) {
+            cost = c;
+            best = t;
         }
     }
-    return {best_zd, best_cost};
+    return best;
 }
 
-// Tile of the ring march over a region of nx x ny x nz cells. FP32 chooses between 64 x 8 and 32 x 16 (512
-// threads, one block per CU) and 16 x 16 (two per CU): all hold 512 cells per CU. The wide blocks read
-// fewer halo cells and parts of cache lines, and their two waves per SIMD cannot drift apart in z,
-// which is what counts once the fields outgrow the caches: at 512^3 16 x 16 blocks move 24 GB of HBM
-// traffic per launch (their neighbours' halo lines have left L2 when they come to them) and take
-// 4.4 ms, 64 x 8 ones 14 GB and 3.58 ms, 32 x 16 ones 3.68; 256^3 0.528 / 0.474 ms, 192 x 160 x 128 127 /
-// 118 us, 128^3 58.1 / 56.9 us. Below that the narrow block's finer grain is worth more (96^3 31.0 / 37.8
-// us, 32 x 16 33.6). Above, the tiles that cover the region at the least cost: 16 x 16 against 32 x 16
-// 352^3 1619 / 1255 us, 224^3 402 / 356, 160^3 137 / 126, 416 x 96 x 96 126 / 118.
-//
-// FP64 (256 columns a block) chooses between 16 x 16 and 32 x 8, which takes 2 to 3 % longer on what both
-// cover alike (128^3 121 / 118 us, 512^3 7.41 / 7.30 ms), by the cost of their z-chunks: 150 x 33 x 110 (30
-// or 25 tiles) 47.2 / 42.5 us, 160 x 40 x 200 76.9 / 69.3; 64 x 24 x 64 (8 or 6, all resident either way)
-// 16.0 / 17.4.
-static int2
-ring_tile(int nx, int ny, int nz)
-{
-    const int2 narrow = make_int2(16, 16);
-#if AC_DOUBLE_PRECISION == 1
-    const int2 flat = make_int2(32, 8);
-    return 1.03 * ring_plan(flat, nx, ny, nz).cost < ring_plan(narrow, nx, ny, nz).cost ? flat : narrow;
-#else
-    if ((long)nx * ny * nz < 1L << 21)
-        return narrow;
-    auto up = [](long n, long t) { return (n + t - 1) / t * t; };
-    auto of = [&](int2 t, long cost) { return up(nx, t.x) * up(ny, t.y) * cost; }; // cost per cell of the tiles
-    const int2 flat = make_int2(64, 8), tall = make_int2(32, 16);
-    const int2 wide = of(tall, 103) < of(flat, 100) ? tall : flat;
-    return of(wide, wide.x == 32 ? 103 : 100) < of(narrow, 112) ? wide : narrow;
-#endif
-}
-
-// z-depth of the ring march over nx x ny x nz cells (0: whole columns).
+// z-depth of the ring march over nx x ny x nz cells (0: whole columns): equal chunks, which keep each XCD's
+// contiguous block range equally loaded, at the least cost in any tile; ring_tile finds that tile again.
 static int
 ring_z_depth(int nx, int ny, int nz)
 {
-    const int zd = ring_plan(ring_tile(nx, ny, nz), nx, ny, nz).zdepth;
-    return zd >= nz ? 0 : zd;
+    int best    = nz;
+    double cost = INFINITY;
+    for (const RingTile& t : kRingTiles) {
+        if (!ring_tile_fits(t, nx, ny, nz))
+            continue;
+        const long cols  = (long)((nx + t.x - 1) / t.x) * ((ny + t.y - 1) / t.y);
+        const long slots = (AC_DOUBLE_PRECISION || t.x * t.y == 512 ? 1L : 2L) * current_cu_count();
+        const long kfill = std::max(1L, (slots + cols - 1) / cols);
+        const int kmax   = (int)std::min(std::max(12L, 4 * kfill), (long)nz);
+        for (int k = 1; k <= kmax; ++k) {
+            const int zd   = (nz + k - 1) / k;
+            const double c = ring_cost(t, nx, ny, nz, zd);
+            if (c < cost) {
+                cost = c;
+                best = zd;
+            }
+        }
+    }
+    return best >= nz ? 0 : best;
 }
 
 AcKernelConfig
@@ -1882,7 +1901,7 @@ template <bool COMP>
 static hipError_t
 launch_ring_tile(const SubstepArgs& a, int zdepth, hipStream_t stream)
 {
-    const int2 tile = ring_tile(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z);
+    const RingTile tile = ring_tile(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z, zdepth);
 #if AC_DOUBLE_PRECISION == 0
     if (tile.x == 64)
         return launch_ring<64, 8, COMP>(a, zdepth, stream);
