@@ -39,9 +39,11 @@
 //  variant 23: variant 17 loading each plane straight into its ring slot (direct-to-LDS loads).
 //  variants 5, 6: the lean z-march with a cell-major LDS ring (FP32; kept for comparison).
 //  variant 19 (FP32) and variant 8 on 16 x 16 tiles in FP64, the defaults: the ring march
-//      (solve_ring.h); variant 24: the FP32 ring march in 64 x 8 blocks whatever the box. The ring
-//      march can read the periodic images of the ghost cells (SubstepArgs::wrap), used by the
-//      whole-step entry points of a periodic box where that is the faster form.
+//      (solve_ring.h, solve_pair.h) in the tile that costs the region least (ring_tile); variant 24:
+//      the ring march in the tile that the configuration names (FP32 64 x 8 or 32 x 16, FP64 32 x 8),
+//      whatever the region. The defaults can read the periodic images of the ghost cells
+//      (SubstepArgs::wrap), used by the whole-step entry points of a periodic box where that is the
+//      faster form.
 #include "physics.h"
 
 #include <algorithm>
@@ -1591,6 +1593,9 @@ constexpr ConfigEntry kConfigs[] = {
     {8, 16, 16},
 #if AC_DOUBLE_PRECISION == 0
     {24, 64, 8},
+    {24, 32, 16},
+#else
+    {24, 32, 8},
 #endif
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
@@ -1899,19 +1904,27 @@ default_kernel_config(int nx, int ny, int nz)
 
 template <bool COMP>
 static hipError_t
-launch_ring_tile(const SubstepArgs& a, int zdepth, hipStream_t stream)
+launch_ring_in(int tile_x, const SubstepArgs& a, int zdepth, hipStream_t stream)
 {
-    const RingTile tile = ring_tile(a.end.x - a.start.x, a.end.y - a.start.y, a.end.z - a.start.z, zdepth);
 #if AC_DOUBLE_PRECISION == 0
-    if (tile.x == 64)
+    if (tile_x == 64)
         return launch_ring<64, 8, COMP>(a, zdepth, stream);
-    if (tile.x == 32)
+    if (tile_x == 32)
         return launch_ring<32, 16, COMP>(a, zdepth, stream);
 #else
-    if (tile.x == 32)
+    if (tile_x == 32)
         return launch_ring<32, 8, COMP>(a, zdepth, stream);
 #endif
     return launch_ring<16, 16, COMP>(a, zdepth, stream);
+}
+
+// The ring march in the tile that the configuration names (variant 24) or the one that ring_tile chooses.
+template <bool COMP>
+static hipError_t
+launch_ring_tile(const AcKernelConfig& c, const SubstepArgs& a, int zdepth, hipStream_t stream)
+{
+    const int nx = a.end.x - a.start.x, ny = a.end.y - a.start.y, nz = a.end.z - a.start.z;
+    return launch_ring_in<COMP>(c.variant == 24 ? c.tile_x : ring_tile(nx, ny, nz, zdepth).x, a, zdepth, stream);
 }
 
 hipError_t
@@ -1925,7 +1938,7 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
     if (a.cin[0] != nullptr) {
         // compensated integration: the ring march with the two error terms, z-depth from `c`
         const int zd = c.variant >= 1 ? c.z_depth : 0;
-        return launch_ring_tile<true>(a, zd, stream);
+        return launch_ring_tile<true>(c, a, zd, stream);
     }
 #define AC_DIRECT(TX, TY)                                                                          \
     if (c.variant == 0 && c.tile_x == TX && c.tile_y == TY)                                        \
@@ -2006,9 +2019,9 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 5, true, true, 7, true>,
                                           a, c.z_depth, stream);
     if (c.variant == 19 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_ring_tile<false>(a, c.z_depth, stream);
-    if (c.variant == 24 && c.tile_x == 64 && c.tile_y == 8)
-        return launch_ring<64, 8, false>(a, c.z_depth, stream);
+        return launch_ring_tile<false>(c, a, c.z_depth, stream);
+    if (c.variant == 24 && ((c.tile_x == 64 && c.tile_y == 8) || (c.tile_x == 32 && c.tile_y == 16)))
+        return launch_ring_tile<false>(c, a, c.z_depth, stream);
     if (c.variant == 22 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 2, 4, true, false, 7, true>,
                                           a, c.z_depth, stream);
@@ -2019,8 +2032,8 @@ launch_substep(const AcKernelConfig& c, const SubstepArgs& a, hipStream_t stream
             stream);
 #endif
 #if AC_DOUBLE_PRECISION == 1
-    if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16)
-        return launch_ring_tile<false>(a, c.z_depth, stream);
+    if ((c.variant == 8 && c.tile_x == 16 && c.tile_y == 16) || (c.variant == 24 && c.tile_x == 32 && c.tile_y == 8))
+        return launch_ring_tile<false>(c, a, c.z_depth, stream);
 #else
     if (c.variant == 8 && c.tile_x == 16 && c.tile_y == 16)
         return launch_zmarch_grid<16, 16>(solve_zlean<16, 16, 1, 4, true, true>, a,

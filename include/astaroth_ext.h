@@ -92,10 +92,11 @@ AcResult acDeviceIntegrateStepGraph(const Device device, const Stream stream, co
  * variants 17, 22: variants 16 and 10 reading each field's LDS stencil window through one pinned
  *            base register (FP32).
  * variant 19: the ring march (FP32 default): cross derivatives half scattered and half gathered, one
- *            barrier per plane. Over regions of 2^21 cells or more that 64 x 8 or 32 x 16 blocks
- *            cover without much waste it runs in such blocks of 512 threads instead of 16 x 16
- *            ones; the results are the same bit for bit.
- * variant 24: the ring march in 64 x 8 blocks over any region (FP32).
+ *            barrier per plane. Variant 19 and FP64's variant 8 on 16 x 16 tiles run in other blocks
+ *            where these cost the region less: FP32 regions of 2^21 cells or more in 64 x 8 or 32 x 16
+ *            blocks of 512 threads, FP64 regions in 32 x 8 ones; the results are the same bit for bit.
+ * variant 24: the ring march in the tile named, 64 x 8 or 32 x 16 (FP32), 32 x 8 (FP64), over any
+ *            region.
  * variant 23: variant 17 with each plane loaded straight into its ring slot by direct-to-LDS
  *            loads (no staging registers or LDS writes; FP32). */
 typedef struct {
@@ -126,8 +127,9 @@ AcResult acDeviceTimestepCFL(const Device device, const Stream stream, double* d
  * a second buffer (two more buffer sets, allocated and zeroed here) and each substep adds its
  * increment with an error-free two-sum: u_out + c_out = u_in + d exactly, where d includes
  * c_in. The right-hand side still reads the rounded state only. Loads, sets and randomisations
- * of a field reset its compensation to zero. The substep then always uses the ring march (the
- * default), with the configuration's z_depth. enable == 0 frees the buffers. */
+ * of a field reset its compensation to zero. The substep then always uses the ring march, with the
+ * configuration's z_depth, in the tile that costs the region least or, with variant 24, the one named.
+ * enable == 0 frees the buffers. */
 AcResult acDeviceSetCompensatedIntegration(const Device device, const int enable);
 
 /* ---- Synthetic initial conditions ----
