@@ -1286,9 +1286,10 @@ acDeviceTimeKernelConfig(const Device device, const AcKernelConfig config, const
     return time_config(device, config, iters);
 }
 
-// ref device.cc:83-98 / integration.cuh:130-215. Sweeps every compiled tile shape and, for the
-// z-march variants, z-depths below n_z plus n_z itself; keeps the fastest substep. Overwrites the
-// `out` buffers (as the reference's sweep does), so call it between full RK3 steps.
+// ref device.cc:83-98 / integration.cuh:130-215. Sweeps the default at its own z-depth, then every
+// compiled tile shape and, for the z-march variants, z-depths below n_z plus n_z itself; keeps the
+// fastest substep. Overwrites the `out` buffers (as the reference's sweep does), so call it between
+// full RK3 steps.
 AcResult
 acDeviceAutoOptimize(const Device device)
 {
@@ -1306,10 +1307,15 @@ acDeviceAutoOptimize(const Device device)
     const long cells = (long)nx_of(device) * ny_of(device) * nz_of(device);
     const int iters  = cells >= (1L << 24) ? 3 : 5;
     AcKernelConfig best = default_kernel_config(nx_of(device), ny_of(device), nz_of(device));
-    float best_ms       = INFINITY;
     // untimed launches first, so that the first configuration timed does not pay for the clocks
     // ramping up from idle
     (void)time_config(device, best, 4 * iters);
+    // the default's own depth, which the cuts below need not hold (384 x 390 x 1009 in FP32: six chunks, 4.26 ms
+    // a launch, 4.50 in four and 4.64 in eight; 256 x 2 x 1024 in FP64: 32 chunks, 96 us, the best of the
+    // others 184)
+    float best_ms = time_config(device, best, iters);
+    if (!(best_ms > 0))
+        best_ms = INFINITY;
     // z-depths: powers of two for variant 1, whole rounds of the unrolled 8-plane loop for
     // variant 13, and for the other lean marches (whose plane loop ends with a partial round)
     // equal chunks: the box's depth cut in 2, 3, 4 or 8
