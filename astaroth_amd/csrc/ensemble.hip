@@ -453,10 +453,14 @@ apply(Ensemble e, const Candidate& c)
 
 // The z-depths of a tile shape by decreasing promise: the work of the busiest block after the dealing,
 // for columns cut at 2 to 128 planes and whole ones. Fewer, longer items save prologues; more, shorter
-// ones fill the chip and leave less of a tail. Leaves the ensemble at the first. None, without dealing,
-// where even an even deal of whole columns would take more than `limit`.
+// ones fill the chip and leave less of a tail. A depth is not dealt where even an equal share of its work
+// takes over MARGIN times `least` or the best so far: the tuner would not time it (with all of them dealt
+// seven ensembles of 12 mixed boxes took 79 ms to create, without 47). Leaves the ensemble at the first, where
+// there is one.
+constexpr double MARGIN = 1.1;
+
 AcResult
-rank_depths(Ensemble e, int tile_x, int tile_y, double limit, std::vector<Candidate>* ranked)
+rank_depths(Ensemble e, int tile_x, int tile_y, double least, std::vector<Candidate>* ranked)
 {
     AC_HIP_CHECK(hipSetDevice(e->id));
     e->tile_x         = tile_x;
@@ -470,23 +474,28 @@ rank_depths(Ensemble e, int tile_x, int tile_y, double limit, std::vector<Candid
     AC_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->id));
     const double per_cu = (double)slots / cus;
     ranked->clear();
-    double even = 0;
-    for (const AcMeshInfo& i : e->info) {
-        const int3 n = dims_of(i);
-        even += (double)plane_cost(box_tiling(launch, n), n) * (PROLOGUE + n.z) / cus;
-    }
-    if (even > limit)
-        return AC_SUCCESS;
+    std::map<int, int> last;
     for (const int depth : {1 << 30, 128, 96, 64, 48, 32, 24, 16, 12, 8, 6, 4, 2}) {
         const std::map<int, int> cut = equal_parts(e, depth);
-        if (!ranked->empty() && cut == ranked->back().class_depth)
+        if (cut == last)
+            continue;
+        last        = cut;
+        double even = 0;
+        for (const AcMeshInfo& i : e->info) {
+            const int3 n = dims_of(i);
+            even += (double)plane_cost(box_tiling(launch, n), n) * (PROLOGUE * tiles(n.z, cut.at(n.z)) + n.z) / cus;
+        }
+        if (even > MARGIN * least)
             continue;
         e->class_depth = cut;
         const Deal d   = deal_items(e, launch, slots);
         ranked->push_back({tile_x, tile_y, cut, d.makespan * per_cu});
+        least = std::min(least, d.makespan * per_cu);
         if (d.items.size() > 32 * (size_t)slots)
             break; // shorter items only cost more
     }
+    if (ranked->empty())
+        return AC_SUCCESS;
     std::stable_sort(ranked->begin(), ranked->end(), [](const Candidate& a, const Candidate& b) { return a.time < b.time; });
     apply(e, ranked->front());
     return AC_SUCCESS;
@@ -743,13 +752,15 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     AC_HIP_CHECK(hipMalloc((void**)&e->d_results, (size_t)nboxes * NDIAG * sizeof(double)));
     AC_HIP_CHECK(hipMemset(e->d_results, 0, (size_t)nboxes * NDIAG * sizeof(double)));
     AC_HIP_CHECK(hipHostMalloc((void**)&e->h_results, (size_t)nboxes * NDIAG * sizeof(double)));
-    std::vector<Candidate> ranked;
-    if (rank_depths(e, 16, 16, INFINITY, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
-        return AC_FAILURE;
-    // Tile shape and z-depths measured on this composition, as Devices tune at creation; AC_AUTOTUNE=0
-    // keeps 16 x 16 tiles at the first depths.
+    // Tile shape and z-depths measured on this composition, as Devices tune at creation; with
+    // AC_AUTOTUNE=0 16 x 16 tiles (or the wide ones of launch_shape) at the depths ranked first.
     const char* tune = getenv("AC_AUTOTUNE");
-    if (!(tune && tune[0] == '0') && acEnsembleAutoOptimize(e) != AC_SUCCESS)
+    if (tune && tune[0] == '0') {
+        std::vector<Candidate> ranked;
+        if (rank_depths(e, 16, 16, INFINITY, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
+            return AC_FAILURE;
+    }
+    else if (acEnsembleAutoOptimize(e) != AC_SUCCESS)
         return AC_FAILURE;
     AC_HIP_CHECK(hipDeviceSynchronize());
     *ensemble = e;
@@ -838,7 +849,7 @@ acEnsembleAutoOptimize(Ensemble e)
     double least = INFINITY;
     for (const int2 tile : {make_int2(16, 16), make_int2(16, 8), make_int2(32, 4)}) {
         std::vector<Candidate> ranked;
-        if (rank_depths(e, tile.x, tile.y, 1.1 * least, &ranked) != AC_SUCCESS)
+        if (rank_depths(e, tile.x, tile.y, least, &ranked) != AC_SUCCESS)
             return AC_FAILURE;
         if (ranked.empty())
             continue;
@@ -846,7 +857,7 @@ acEnsembleAutoOptimize(Ensemble e)
         candidates.insert(candidates.end(), ranked.begin(), ranked.begin() + std::min<size_t>(ranked.size(), 4));
     }
     candidates.erase(std::remove_if(candidates.begin(), candidates.end(),
-                                    [=](const Candidate& c) { return c.time > 1.1 * least; }),
+                                    [=](const Candidate& c) { return c.time > MARGIN * least; }),
                      candidates.end());
     float best  = INFINITY;
     size_t keep = 0;
