@@ -114,6 +114,10 @@ hipError_t launch_substep_batch(int tile_x, int tile_y, int step, const SubstepA
 int kernel_config_count();
 AcKernelConfig kernel_config_at(int index);
 AcKernelConfig default_kernel_config(int nx, int ny, int nz);
+// Whether the configuration is, over this region, the launch of the default variant at the same z-depth by
+// another name (variant 24 in the tile that the default takes there). The default is to be preferred
+// then: it takes the tile that suits any other region, and can read images.
+bool is_default_launch(const AcKernelConfig& config, int nx, int ny, int nz);
 
 // Periodic fill of the ghost cells inside [start, end) of `nfields` buffers (boundconds.hip).
 hipError_t launch_periodic_fill(AcReal* const* fields, int nfields, int nx, int ny, int nz,

@@ -1331,7 +1331,7 @@ acDeviceAutoOptimize(const Device device)
         const int ndepth  = c.variant == 0 ? 1 : c.variant == 1 ? 6 : 5;
         for (int di = 0; di < ndepth; ++di) {
             c.z_depth = c.variant == 0 ? 0 : depths[di];
-            if (c.z_depth >= nz_of(device))
+            if (c.z_depth >= nz_of(device) || is_default_launch(c, nx_of(device), ny_of(device), nz_of(device)))
                 continue;
             const float ms = time_config(device, c, iters);
             if (ms > 0 && ms < best_ms) {

@@ -1902,6 +1902,15 @@ default_kernel_config(int nx, int ny, int nz)
     return c;
 }
 
+bool
+is_default_launch(const AcKernelConfig& c, int nx, int ny, int nz)
+{
+    if (c.variant != 24)
+        return false;
+    const RingTile t = ring_tile(nx, ny, nz, c.z_depth);
+    return t.x == c.tile_x && t.y == c.tile_y;
+}
+
 template <bool COMP>
 static hipError_t
 launch_ring_in(int tile_x, const SubstepArgs& a, int zdepth, hipStream_t stream)
