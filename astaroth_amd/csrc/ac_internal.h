@@ -177,8 +177,8 @@ struct device_s {
     double* reduce_partials;
     double* reduce_scratch; // this GPU's copy of the library's reduction scratch array
     double* reduce_result; // pinned host memory
-    double* diag_partials;      // acDeviceDiagnostics: per-block partials, results, pinned copy
-    double* diag_result; // pinned host memory
+    double* diag_partials; // acDeviceDiagnostics: per-block partials, in device memory,
+    double* diag_result;   // and results, in pinned host memory
     AcKernelConfig kernel_config;
     // periodic steps read the ghost cells' images where the configuration has such a build
     // (default by size, measured by acDeviceAutoOptimize, set by acDeviceSetReadPeriodicImages)

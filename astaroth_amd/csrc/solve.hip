@@ -1743,11 +1743,11 @@ default_reads_images(int nx, int ny, int nz)
 {
     // Reading images saves the three fills of a step but slows the launches down as the box grows
     // (the far-side halo and plane reads). Per step, images against fills (ms, sustained):
-    //   FP32  128^3 0.176 / 0.201   256^3 1.45 / 1.47   384^3 4.93 / 5.04   448^3 7.91 / 8.06
-    //         512^3 11.80 / 11.40
-    //   FP64  128^3 0.351 / 0.400   256^3 2.65 / 2.79   384^3 9.40 / 9.71   512^3 21.6 / 22.1
-    // so images below 512^3 cells, in FP64 too: its crossover lies higher, but a caller of a 512^3 box
-    // has found its ghosts filled by the step.
+    //   FP32  256^3 1.41 / 1.42   384^3 4.83 / 4.92   448^3 7.73 / 7.85   480^3 10.03 / 9.99
+    //         512^3 11.55 / 11.30   640^3 22.3 / 22.6   768^3 41.3 / 38.0   93 x 1188 x 1219 13.2 / 14.7
+    //   FP64  256^3 2.62 / 2.75   384^3 9.28 / 9.56   512^3 21.4 / 22.0   640^3 43.3 / 43.5   768^3 76.0 / 74.4
+    // so images below 512^3 cells. Above, FP32 depends on the shape and FP64 gains up to 3 % from images until
+    // about 640^3: the tuner measures both forms.
     return (double)nx * ny * nz < 512.0 * 512.0 * 512.0;
 }
 
@@ -1797,7 +1797,7 @@ current_cu_count()
 // per CU): all hold 512 cells per CU. The wide blocks read fewer halo cells and parts of cache lines,
 // and their two waves per SIMD cannot drift apart in z, which is what counts once the fields outgrow
 // the caches: at 512^3 16 x 16 blocks move 24 GB of HBM traffic per launch (their neighbours' halo lines
-// have left L2 when they come to them) and take 4.4 ms, 64 x 8 ones 14 GB and 3.62 ms. FP64 (256 columns a
+// have left L2 when they come to them) and take 4.4 ms, 64 x 8 ones 12.5 GB and 3.54 ms. FP64 (256 columns a
 // block) has 16 x 16 and 32 x 8, which takes 2 to 3 % longer on what both cover alike (128^3 121 / 118 us,
 // 512^3 7.41 / 7.30 ms).
 struct RingTile {

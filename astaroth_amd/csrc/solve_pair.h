@@ -14,10 +14,11 @@
 //
 // What bounds it: a lone block takes 2.55 us a plane, about 45 % of it VALU issue and 45 % LDS, which the
 // barriers keep from overlapping fully (offsetting the groups by half a plane gained 2 % on a full chip
-// and cost a four-plane column 15 %). On a full chip the clock drops from 2.4 to 2.2 GHz and the fields
-// stream at 3.7 TB/s, 80 % of what a plain copy reaches. Per launch, sustained (us), one thread per
-// column -> this: 32^3 16.5 -> 13.0, 64^3 26.7 -> 23.5, 150 x 33 x 110 65 -> 48, 128^3 140 -> 123, 256^3
-// 1020 -> 895, 512^3 8160 -> 7240.
+// and cost a four-plane column 15 %). On a full chip the clock drops from 2.4 to 2.0 GHz; at 512^3 a
+// launch of substeps 1 and 2 moves 29.5 GB at 4.0 TB/s, 85 % of what a plain copy of 4 GiB reaches, and
+// substep 0 20.8 GB at 3.3 TB/s. Per launch, sustained, mean of the three substeps (us), one thread per
+// column -> this: 32^3 16.5 -> 12.1, 64^3 26.7 -> 22.0, 150 x 33 x 110 65 -> 42.6, 128^3 140 -> 113, 256^3
+// 1020 -> 867, 512^3 8160 -> 7020.
 #pragma once
 #include "physics.h"
 
@@ -64,8 +65,8 @@ template <int TX, int TY, bool COMP, bool FIRST> struct ZMarchPair {
     };
 
     // The constants of the rates and the update, in vector registers: with the stencils' they exceed
-    // the scalar ones, and what spills is read back lane by lane (78 v_readlane a plane, 24 with
-    // these; 256^3 948 -> 917 us).
+    // the scalar ones, and what spills is read back lane by lane (78 v_readlane a plane; with these 36, in
+    // substep 0 24; 256^3 948 -> 917 us).
     struct Constants {
         AcReal nu_visc, eta, inv_mu0, eta_mu0, inv_cp, gamma_inv_cp, gamma_m1, exp_lnT0, lnrho0, zeta, cs2_sound,
             k_thermal, dt, beta, ab;

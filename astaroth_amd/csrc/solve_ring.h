@@ -17,7 +17,7 @@
 // * Each field's LDS reads are issued before the arithmetic of the field before it, in an order that
 //   scheduling barriers hold. The lean march consumed most of its reads as they were issued: 90 waits
 //   a plane for LDS, now 60, most of them satisfied. With registers to spare from the smaller
-//   pending state this needs no spill (FP32 200 of 256 registers; the same order cost the lean
+//   pending state this needs no spill (FP32 204 of 256 registers; the same order cost the lean
 //   march more in spills than it saved).
 // * The ring rows hold all eight fields of a tile row side by side, so one LDS base register per row
 //   serves every field's x window, and rows a tile row apart start 16 banks apart (16-wide tiles).
@@ -27,10 +27,11 @@
 //   formed with fewer operations (mhd_rates_lean). The vector instruction count is level with the
 //   lean march's (630 a plane in FP32): what it gains is in the waits.
 //
-// What bounds it: the vector pipes are busy 65 to 73 % of the time on boxes that fit the caches (LDS
-// 50 %); at 512^3 the launch moves 14 GB, 85 % of what a plain copy reaches on this card. Per launch,
-// sustained (us), lean march -> this: 32^3 27.9 -> 7.8, 97 x 61 x 75 35.8 -> 26.2, 128^3 74.7 -> 57.9,
-// 256^3 529 -> 456, 512^3 4020 -> 3600.
+// What bounds it: the vector pipes are busy 65 to 75 % of the time (LDS 50 to 57 %). At 512^3 a launch of
+// substeps 1 and 2 moves 13.9 GB at 3.8 TB/s, 81 % of what a plain copy of 4 GiB reaches on this card; substep
+// 0 moves 9.6 GB at 2.9 TB/s and is bound by instruction issue. Per launch, sustained, mean of the three
+// substeps (us), lean march -> this: 32^3 27.9 -> 7.6, 97 x 61 x 75 35.8 -> 25.4, 128^3 74.7 -> 56.2, 256^3
+// 529 -> 447, 512^3 4020 -> 3540.
 #pragma once
 #include "physics.h"
 

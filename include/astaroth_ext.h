@@ -49,7 +49,8 @@ AcResult acDeviceReduceNoAlloc(const Device device, const Stream stream, const R
  * (src/core/node.cc:729-806). With the default kernel configuration (FP32 variant 19, FP64
  * variant 8; 16 x 16 tiles), compensated integration off and n >= 3 on every axis, the substeps
  * can instead read the periodic images of the ghost cells directly and make no fill: by default
- * below 512^3 cells (above, reading them costs more than the fills it saves); acDeviceAutoOptimize measures both forms and keeps the faster, and
+ * below 512^3 cells (above, which form is faster depends on precision and shape, by up to 10 % either
+ * way); acDeviceAutoOptimize measures both forms and keeps the faster, and
  * acDeviceSetReadPeriodicImages overrides the choice. The state ends in `in` without a final
  * fill, as in the reference: its ghost cells are to be filled before they are read. */
 AcResult acDeviceIntegrateStep(const Device device, const Stream stream, const AcReal dt);
