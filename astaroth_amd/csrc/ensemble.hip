@@ -217,14 +217,13 @@ struct ensemble_s {
     size_t base_bytes;
     hipStream_t stream;
     int parity; // number of swaps mod 2: set `parity` holds the current state
-    // batched solve: one tile shape per launch (see launch_shape for 16 x 16); the z-depth of a
-    // box's work items is that of its size class (its column length n_z) when the ensemble chose
-    // it, else z_depth (0: whole columns)
+    // batched solve: one tile shape per launch, 64 x 8 for 512-thread blocks (see wide_tiling); the
+    // z-depth of a box's work items is that of its size class (its column length n_z) when the ensemble
+    // chose it, else z_depth (0: whole columns)
     int tile_x, tile_y, z_depth, nblocks;
     std::map<int, int> class_depth;
     BatchItem* d_items;
     int nitems;
-    int2 launch; // tile shape of the launch
     SubstepArgs* d_args[3][2]; // per (substep, parity), for dt_args
     AcReal dt_args;
     bool args_valid;
@@ -323,13 +322,13 @@ narrow_tiling(int tx, int ty)
     return {tx, ty, 0, weight};
 }
 
-// Tile shape of the launch. In FP32 a 16 x 16 configuration runs 512-thread blocks if their tiles
-// cost less over the whole ensemble (100 boxes of 48^3, which they cover with a third to spare, take
+// Tile shape of the launch of a configuration. In FP32 a 16 x 16 one runs 512-thread blocks if their
+// tiles cost less over the whole ensemble (100 boxes of 48^3, which they cover with a third to spare, take
 // 1.43 ms per step in 16 x 16 tiles and 1.52 in 64 x 8).
 int2
-launch_shape(const Ensemble e)
+launch_shape(const Ensemble e, int tile_x, int tile_y)
 {
-    if (!AC_DOUBLE_PRECISION && e->tile_x == 16 && e->tile_y == 16) {
+    if (!AC_DOUBLE_PRECISION && tile_x == 16 && tile_y == 16) {
         long wide = 0, narrow = 0;
         for (const AcMeshInfo& i : e->info) {
             const int3 n = dims_of(i);
@@ -339,7 +338,7 @@ launch_shape(const Ensemble e)
         if (wide < narrow)
             return make_int2(64, 8);
     }
-    return make_int2(e->tile_x, e->tile_y);
+    return make_int2(tile_x, tile_y);
 }
 
 Tiling
@@ -403,7 +402,7 @@ AcResult
 build_items(Ensemble e)
 {
     AC_HIP_CHECK(hipSetDevice(e->id));
-    const int2 launch = launch_shape(e);
+    const int2 launch = make_int2(e->tile_x, e->tile_y);
     // the persistent grid: one block per resident block slot of the batched kernel
     const int slots = batch_resident_blocks(launch.x, launch.y);
     if (slots < 1)
@@ -417,7 +416,6 @@ build_items(Ensemble e)
     AC_HIP_CHECK(hipMalloc((void**)&e->d_items, d.items.size() * sizeof(BatchItem)));
     AC_HIP_CHECK(hipMemcpy(e->d_items, d.items.data(), d.items.size() * sizeof(BatchItem),
                            hipMemcpyHostToDevice));
-    e->launch  = launch;
     e->nitems  = (int)d.items.size();
     e->nblocks = d.slots;
     return AC_SUCCESS;
@@ -460,14 +458,13 @@ apply(Ensemble e, const Candidate& c)
 constexpr double MARGIN = 1.1;
 
 AcResult
-rank_depths(Ensemble e, int tile_x, int tile_y, double least, std::vector<Candidate>* ranked)
+rank_depths(Ensemble e, int2 launch, double least, std::vector<Candidate>* ranked)
 {
     AC_HIP_CHECK(hipSetDevice(e->id));
-    e->tile_x         = tile_x;
-    e->tile_y         = tile_y;
-    e->z_depth        = 0;
-    const int2 launch = launch_shape(e);
-    const int slots   = batch_resident_blocks(launch.x, launch.y);
+    e->tile_x       = launch.x;
+    e->tile_y       = launch.y;
+    e->z_depth      = 0;
+    const int slots = batch_resident_blocks(launch.x, launch.y);
     if (slots < 1)
         return AC_FAILURE;
     int cus = 0;
@@ -489,7 +486,7 @@ rank_depths(Ensemble e, int tile_x, int tile_y, double least, std::vector<Candid
             continue;
         e->class_depth = cut;
         const Deal d   = deal_items(e, launch, slots);
-        ranked->push_back({tile_x, tile_y, cut, d.makespan * per_cu});
+        ranked->push_back({launch.x, launch.y, cut, d.makespan * per_cu});
         least = std::min(least, d.makespan * per_cu);
         if (d.items.size() > 32 * (size_t)slots)
             break; // shorter items only cost more
@@ -582,7 +579,7 @@ enqueue_step(Ensemble e, int par0)
     // fill; one fill after the last substep leaves every box's ghosts current.
     int par = par0;
     for (int s = 0; s < 3; ++s) {
-        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, s, e->d_args[s][par], e->d_items,
+        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, s, e->d_args[s][par], e->d_items,
                                           e->nitems, e->nblocks, e->stream));
         par = 1 - par;
     }
@@ -608,12 +605,12 @@ time_batch(Ensemble e, int warm, int samples)
     AC_HIP_CHECK(hipEventCreate(&t1));
     const SubstepArgs* args = e->d_args[1][e->parity];
     for (int i = 0; i < warm; ++i)
-        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, 1, args, e->d_items, e->nitems,
+        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, 1, args, e->d_items, e->nitems,
                                           e->nblocks, e->stream));
     float best = INFINITY;
     for (int i = 0; i < samples; ++i) {
         AC_HIP_CHECK(hipEventRecord(t0, e->stream));
-        AC_HIP_CHECK(launch_substep_batch(e->launch.x, e->launch.y, 1, args, e->d_items, e->nitems,
+        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, 1, args, e->d_items, e->nitems,
                                           e->nblocks, e->stream));
         AC_HIP_CHECK(hipEventRecord(t1, e->stream));
         AC_HIP_CHECK(hipEventSynchronize(t1));
@@ -675,9 +672,7 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     for (auto& i : e->info)
         acHostUpdateBuiltinParams(&i);
     e->parity   = 0;
-    // 16 x 16 tiles (or the wide ones of launch_shape) at the z-depths ranked first, until the tuner
-    // (below) measures this composition
-    e->tile_x   = 16;
+    e->tile_x   = 16; // (and chosen below)
     e->tile_y   = 16;
     e->z_depth  = 0;
     e->d_items  = nullptr;
@@ -757,7 +752,7 @@ acEnsembleCreate(const int device_id, const int nboxes, const AcMeshInfo* config
     const char* tune = getenv("AC_AUTOTUNE");
     if (tune && tune[0] == '0') {
         std::vector<Candidate> ranked;
-        if (rank_depths(e, 16, 16, INFINITY, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
+        if (rank_depths(e, launch_shape(e, 16, 16), INFINITY, &ranked) != AC_SUCCESS || build_items(e) != AC_SUCCESS)
             return AC_FAILURE;
     }
     else if (acEnsembleAutoOptimize(e) != AC_SUCCESS)
@@ -807,9 +802,10 @@ acEnsembleSetKernelConfig(Ensemble e, const AcKernelConfig config)
         return AC_FAILURE;
     AC_HIP_CHECK(hipSetDevice(e->id));
     AC_HIP_CHECK(hipStreamSynchronize(e->stream));
-    e->tile_x  = config.tile_x;
-    e->tile_y  = config.tile_y;
-    e->z_depth = config.z_depth;
+    const int2 launch = launch_shape(e, config.tile_x, config.tile_y);
+    e->tile_x         = launch.x;
+    e->tile_y         = launch.y;
+    e->z_depth        = config.z_depth;
     e->class_depth.clear(); // one z-depth for every box
     drop_graphs(e);
     return build_items(e);
@@ -847,9 +843,17 @@ acEnsembleAutoOptimize(Ensemble e)
     // boxes of 32 to 128 cells an edge took 9 ms longer to create with 1.2.
     std::vector<Candidate> candidates;
     double least = INFINITY;
-    for (const int2 tile : {make_int2(16, 16), make_int2(16, 8), make_int2(32, 4)}) {
+    // The 512-thread blocks and 16 x 16 ones are both in the choice (FP32; the one that covers the boxes at
+    // less cost first): with few boxes the rounds of blocks decide (2 boxes of 200^3 1.95 ms per step in 16 x
+    // 16 tiles and 2.07 in 64 x 8, which cover them at 2 % less).
+    std::vector<int2> shapes{launch_shape(e, 16, 16)};
+    if (!AC_DOUBLE_PRECISION)
+        shapes.push_back(shapes[0].x == 64 ? make_int2(16, 16) : make_int2(64, 8));
+    shapes.push_back(make_int2(16, 8));
+    shapes.push_back(make_int2(32, 4));
+    for (const int2 launch : shapes) {
         std::vector<Candidate> ranked;
-        if (rank_depths(e, tile.x, tile.y, least, &ranked) != AC_SUCCESS)
+        if (rank_depths(e, launch, least, &ranked) != AC_SUCCESS)
             return AC_FAILURE;
         if (ranked.empty())
             continue;
@@ -897,8 +901,9 @@ acEnsembleGetKernelConfig(const Ensemble e, AcKernelConfig* config)
     if (!e || !config)
         return AC_FAILURE;
     config->variant = 3;
-    config->tile_x  = e->tile_x;
-    config->tile_y  = e->tile_y;
+    const bool wide = e->tile_x == 64; // not a configuration of its own: 16 x 16 stands for it
+    config->tile_x  = wide ? 16 : e->tile_x;
+    config->tile_y  = wide ? 16 : e->tile_y;
     config->z_depth = e->z_depth;
     return AC_SUCCESS;
 }

@@ -197,11 +197,12 @@ AcResult acEnsembleDestroy(Ensemble ensemble);
 int acEnsembleBoxCount(const Ensemble ensemble);
 /* Batched solve configuration: variant 3, tile 32x4, 16x8 or 16x16, z_depth (0: whole box) for
  * every box (it replaces the ensemble's own per-class z-depths). In FP32, 16x16 stands for blocks of
- * 512 threads in 64x8 or 32x16 tiles where these cover the boxes with little to spare. */
+ * 512 threads in 64x8 or 32x16 tiles where these cover the boxes with little to spare (or where the tuner
+ * found them faster). */
 AcResult acEnsembleSetKernelConfig(Ensemble ensemble, const AcKernelConfig config);
 AcResult acEnsembleGetKernelConfig(const Ensemble ensemble, AcKernelConfig* config);
 /* The ensemble's tuner, run by acEnsembleCreate unless the environment sets AC_AUTOTUNE=0 (then
- * 16 x 16 tiles). For each tile shape the z-depths (columns of every size class in equal parts) are
+ * 16 x 16 tiles). For each tile shape (in FP32 512-thread blocks too) the z-depths (columns of every size class in equal parts) are
  * ranked by the work of the busiest block after the work items are dealt to the resident blocks; the
  * tuner times the batched launch with the first four of each shape that comes within 10 % of the most
  * promising one and keeps the fastest (without it: the first depths). Results are kept per
