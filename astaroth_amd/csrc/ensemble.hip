@@ -594,33 +594,27 @@ valid_dt(AcReal dt)
     return std::isfinite((double)dt) && dt > 0;
 }
 
-// Shortest of `samples` launches of substep 1 of the batched solve over the current work list,
-// after `warm` untimed ones (two of a step's three launches read a previous stage, substep 0 does
-// not). It reads the current set and rewrites the other one, which holds no state between steps.
+// Time of a step's three launches of the batched solve over the current work list. All read the current
+// set and write the other one, which holds no state between steps. The three differ: substep 0 has no
+// previous stage to read, and 16 x 16 blocks gain more by that than 512-thread ones (2 boxes of 200^3: substep 1
+// 0.59 and 0.60 ms, substep 0 0.46 and 0.56).
 float
-time_batch(Ensemble e, int warm, int samples)
+time_solves(Ensemble e)
 {
     hipEvent_t t0, t1;
     AC_HIP_CHECK(hipEventCreate(&t0));
     AC_HIP_CHECK(hipEventCreate(&t1));
-    const SubstepArgs* args = e->d_args[1][e->parity];
-    for (int i = 0; i < warm; ++i)
-        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, 1, args, e->d_items, e->nitems,
-                                          e->nblocks, e->stream));
-    float best = INFINITY;
-    for (int i = 0; i < samples; ++i) {
-        AC_HIP_CHECK(hipEventRecord(t0, e->stream));
-        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, 1, args, e->d_items, e->nitems,
-                                          e->nblocks, e->stream));
-        AC_HIP_CHECK(hipEventRecord(t1, e->stream));
-        AC_HIP_CHECK(hipEventSynchronize(t1));
-        float ms = 0;
-        AC_HIP_CHECK(hipEventElapsedTime(&ms, t0, t1));
-        best = std::min(best, ms);
-    }
+    AC_HIP_CHECK(hipEventRecord(t0, e->stream));
+    for (int s = 0; s < 3; ++s)
+        AC_HIP_CHECK(launch_substep_batch(e->tile_x, e->tile_y, s, e->d_args[s][e->parity], e->d_items,
+                                          e->nitems, e->nblocks, e->stream));
+    AC_HIP_CHECK(hipEventRecord(t1, e->stream));
+    AC_HIP_CHECK(hipEventSynchronize(t1));
+    float ms = 0;
+    AC_HIP_CHECK(hipEventElapsedTime(&ms, t0, t1));
     AC_HIP_CHECK(hipEventDestroy(t0));
     AC_HIP_CHECK(hipEventDestroy(t1));
-    return best;
+    return ms;
 }
 
 // Tuned choices per ensemble composition (device, box sizes in order), kept for the process.
@@ -865,12 +859,12 @@ acEnsembleAutoOptimize(Ensemble e)
                      candidates.end());
     float best  = INFINITY;
     size_t keep = 0;
-    for (int round = 0; round < 2; ++round) // twice: the clocks still rise during the first
+    for (int round = 0; round < 3; ++round) // the clocks still rise during the first
         for (size_t i = 0; i < candidates.size(); ++i) {
             apply(e, candidates[i]);
             if (build_items(e) != AC_SUCCESS)
                 return AC_FAILURE;
-            const float ms   = time_batch(e, 1, 2);
+            const float ms   = time_solves(e);
             const bool other = candidates[i].tile_x != candidates[keep].tile_x || candidates[i].tile_y != candidates[keep].tile_y;
             if (round > 0 && ms < (other ? 0.98f : 1.f) * best) { // (the timings scatter by 1 to 2 %)
                 best = ms;
