@@ -204,7 +204,7 @@ AcResult acEnsembleGetKernelConfig(const Ensemble ensemble, AcKernelConfig* conf
 /* The ensemble's tuner, run by acEnsembleCreate unless the environment sets AC_AUTOTUNE=0 (then
  * 16 x 16 tiles). For each tile shape (in FP32 512-thread blocks too) the z-depths (columns of every size class in equal parts) are
  * ranked by the work of the busiest block after the work items are dealt to the resident blocks; the
- * tuner times the batched launch with the first four of each shape that comes within 10 % of the most
+ * tuner times a step's three launches with the first four of each shape that comes within 10 % of the most
  * promising one and keeps the fastest (without it: the first depths). Results are kept per
  * composition (device and box sizes) for the process. acEnsembleBoxZDepth gives a box's output planes
  * per work item (0: whole columns). */
